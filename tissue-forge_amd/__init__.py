@@ -635,10 +635,10 @@ class Engine:
 
     def particles(self):
         n = self.nparts
-        cid = np.zeros(n, dtype=np.int32)
-        x = np.zeros((n, 3))
-        v = np.zeros((n, 3))
-        f = np.zeros((n, 4))
+        cid = np.empty(n, dtype=np.int32)
+        x = np.empty((n, 3))
+        v = np.empty((n, 3))
+        f = np.empty((n, 4))
         sp = np.zeros((n, max(self.nspecies, 1)))
         q = np.zeros((n, max(self.nspecies, 1)))
         _check(lib().tfg_read_particles(self._h, cid.ctypes.data_as(_i32p), _dptr(x), _dptr(v), _dptr(f),
@@ -650,7 +650,7 @@ class Engine:
         return out
 
     def positions(self):
-        xg = np.zeros((self.nparts, 3))
+        xg = np.empty((self.nparts, 3))
         _check(lib().tfg_read_positions(self._h, _dptr(xg)))
         return xg
 

@@ -122,7 +122,26 @@ struct DeviceEnsemble {
     long long *d_step = nullptr;
     int *d_err = nullptr;
 
+    // Readback: a pinned buffer and an event per reading thread.
+    struct ReadSlot {
+        unsigned char *ptr = nullptr;
+        size_t bytes = 0;
+        hipEvent_t done = nullptr;
+    };
+    ReadSlot read_slot[8];
+    // keep_reads: the state of each member at its last read, by id on the
+    // device (kept, with its energies), for host engines that leave the
+    // ensemble without a download.
+    bool keep_reads = false;
+    ReadRows kept;
+    double *kept_energy = nullptr;
+    std::vector<char> kept_sys;
+
     ~DeviceEnsemble() {
+        for (ReadSlot &r : read_slot) {
+            if (r.ptr) (void)hipHostFree(r.ptr);
+            if (r.done) (void)hipEventDestroy(r.done);
+        }
         for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
         if (graph) (void)hipGraphExecDestroy(graph);
         for (int k = 0; k < nev; k++) (void)hipEventDestroy(ev[k]);
@@ -145,6 +164,7 @@ struct DeviceEnsemble {
 };
 
 int launch_error(const char *what);
+Energies energies_of(const double *e);
 
 template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy);
 
@@ -154,6 +174,11 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy);
 // state is not changed.  Allocates no device memory, creates no stream or
 // event; runs on the null stream and returns after it has drained.
 int ensemble_force_arena(Engine *e, int precision, void *arena, size_t cap, double *f, Energies *en);
+
+// Readback (readback.hip): system s from the device into its host engine's
+// particles, and for keep_reads its state kept on the device and put back.
+int read_into_engine(DeviceEnsemble *E, int s);
+int restore_kept(DeviceEnsemble *E);
 
 // Binning: scan of the cell counts, placement, per-cell order, permutation
 // of buffer B into buffer A.  Cell counts come from the previous advance.

@@ -11,6 +11,18 @@ namespace tfg {
 
 int energy_tile();
 
+// A system's device sums: nonbonded, virial, kinetic, bonds, angles.
+Energies energies_of(const double *e) {
+    Energies out;
+    out.epot_nonbond = e[0];
+    out.virial = e[1];
+    out.ekin = e[2];
+    out.epot_bond = e[3];
+    out.epot_angle = e[4];
+    out.epot = e[0] + e[3] + e[4];
+    return out;
+}
+
 int launch_error(const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(TFG_E_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
@@ -762,8 +774,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
 
 int ensemble_destroy(DeviceEnsemble *E, bool download) {
     if (!E) return TFG_OK;
-    int rc = TFG_OK;
-    if (download) rc = ensemble_download(E);
+    const int rc = download ? ensemble_download(E) : restore_kept(E);
     for (Engine *e : E->engines) {
         e->device = nullptr;
         e->device_index = -1;
@@ -772,68 +783,25 @@ int ensemble_destroy(DeviceEnsemble *E, bool download) {
     return rc;
 }
 
-template <typename real> static int download_t(DeviceEnsemble *E, int only) {
-    using v4 = typename V<real>::v4;
-    int rs;
-    if ((rs = run_sync<real>(E, make_params<real>(E, 0), true)) != TFG_OK) return rs;
-    TFG_HIP(hipStreamSynchronize(E->stream));
-    const int np = E->np, S = E->S;
-    std::vector<v4> hpos(np), hvel(np), hf(np);
-    std::vector<int4> hmeta(np);
-    std::vector<int> hslot(np);
-    std::vector<real> hsp((size_t)np * S), hq((size_t)np * S);
-    // Current state: buffer B (the state after the last update, in A's order).
-    TFG_HIP(hipMemcpy(hpos.data(), E->pos[1], sizeof(v4) * np, hipMemcpyDeviceToHost));
-    TFG_HIP(hipMemcpy(hvel.data(), E->vel[1], sizeof(v4) * np, hipMemcpyDeviceToHost));
-    TFG_HIP(hipMemcpy(hmeta.data(), E->meta[1], sizeof(int4) * np, hipMemcpyDeviceToHost));
-    TFG_HIP(hipMemcpy(hf.data(), E->force, sizeof(v4) * np, hipMemcpyDeviceToHost));
-    TFG_HIP(hipMemcpy(hslot.data(), E->slot_of, sizeof(int) * np, hipMemcpyDeviceToHost));
-    if (S > 0) {
-        TFG_HIP(hipMemcpy(hsp.data(), E->sp[1], sizeof(real) * hsp.size(), hipMemcpyDeviceToHost));
-        TFG_HIP(hipMemcpy(hq.data(), E->qq[1], sizeof(real) * hq.size(), hipMemcpyDeviceToHost));
-    }
+static int download(DeviceEnsemble *E, int only) {
     long long steps = 0;
+    std::vector<double> en(static_cast<size_t>(5) * E->nsys);
+    TFG_HIP(hipStreamSynchronize(E->stream));
     TFG_HIP(hipMemcpy(&steps, E->d_step, sizeof(steps), hipMemcpyDeviceToHost));
+    TFG_HIP(hipMemcpy(en.data(), E->d_energy, sizeof(double) * en.size(), hipMemcpyDeviceToHost));
     for (int s = 0; s < E->nsys; s++) {
         if (only >= 0 && s != only) continue;
-        Engine &e = *E->engines[s];
-        const SysDesc &d = E->sys[s];
-        for (int p = 0; p < d.np; p++) {
-            const int slot = hslot[d.p_off + p];
-            HostParticle &hp = e.parts[p];
-            hp.x[0] = static_cast<double>(hpos[slot].x) + d.foff[0];
-            hp.x[1] = static_cast<double>(hpos[slot].y) + d.foff[1];
-            hp.x[2] = static_cast<double>(hpos[slot].z) + d.foff[2];
-            hp.v[0] = hvel[slot].x;
-            hp.v[1] = hvel[slot].y;
-            hp.v[2] = hvel[slot].z;
-            hp.f[0] = hf[slot].x;
-            hp.f[1] = hf[slot].y;
-            hp.f[2] = hf[slot].z;
-            hp.f[3] = hf[slot].w;
-            hp.cid = hmeta[slot].z - d.cell_off;
-            hp.flags = static_cast<uint32_t>(hmeta[slot].x) >> 16;
-            for (int k = 0; k < e.nspecies; k++) {
-                e.species[(size_t)p * e.nspecies + k] = hsp[(size_t)k * np + slot];
-                e.species_q[(size_t)p * e.nspecies + k] = hq[(size_t)k * np + slot];
-            }
-        }
-        e.time = d.time0 + steps;
-        Energies en;
-        int rc = ensemble_energies(E, s, &en);
+        const int rc = read_into_engine(E, s);
         if (rc != TFG_OK) return rc;
-        e.energies = en;
+        E->engines[s]->time = E->sys[s].time0 + steps;
+        E->engines[s]->energies = energies_of(&en[static_cast<size_t>(5) * s]);
     }
     return TFG_OK;
 }
 
-int ensemble_download(DeviceEnsemble *E) {
-    return E->precision == PREC_MIXED ? download_t<float>(E, -1) : download_t<double>(E, -1);
-}
+int ensemble_download(DeviceEnsemble *E) { return download(E, -1); }
 
-int ensemble_download_one(DeviceEnsemble *E, int sys) {
-    return E->precision == PREC_MIXED ? download_t<float>(E, sys) : download_t<double>(E, sys);
-}
+int ensemble_download_one(DeviceEnsemble *E, int sys) { return download(E, sys); }
 
 template <typename real> static int step_t(DeviceEnsemble *E, int nsteps, bool use_graph) {
     int rc;
@@ -1054,12 +1022,7 @@ int ensemble_energies(DeviceEnsemble *E, int s, Energies *out) {
     double e[5];
     TFG_HIP(hipStreamSynchronize(E->stream));
     TFG_HIP(hipMemcpy(e, E->d_energy + 5 * s, sizeof(e), hipMemcpyDeviceToHost));
-    out->epot_nonbond = e[0];
-    out->virial = e[1];
-    out->ekin = e[2];
-    out->epot_bond = e[3];
-    out->epot_angle = e[4];
-    out->epot = e[0] + e[3] + e[4];
+    *out = energies_of(e);
     return TFG_OK;
 }
 

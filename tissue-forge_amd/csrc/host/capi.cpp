@@ -707,8 +707,17 @@ int tfg_read_particles(tfg_engine *h, int32_t *cid, double *x, double *v, double
                        double *species_q) {
     if (!h) return set_error(TFG_E_INVALIDARG, "null engine");
     if (h->e.device) {
-        int rc = ensemble_download_one(h->e.device, h->e.device_index);
-        if (rc != TFG_OK) return rc;
+        ReadRows out;
+        out.x = x;
+        out.v = v;
+        out.f = f;
+        out.cid = cid;
+        out.ns = h->e.nspecies;
+        if (out.ns > 0) {
+            out.sp = species;
+            out.q = species_q;
+        }
+        TFG_GUARD(return ensemble_read(h->e.device, h->e.device_index, out));
     }
     const Engine &e = h->e;
     const int n = static_cast<int>(e.parts.size());
@@ -733,8 +742,9 @@ int tfg_read_particles(tfg_engine *h, int32_t *cid, double *x, double *v, double
 int tfg_read_positions(tfg_engine *h, double *xg) {
     if (!h || !xg) return set_error(TFG_E_INVALIDARG, "null argument");
     if (h->e.device) {
-        int rc = ensemble_download_one(h->e.device, h->e.device_index);
-        if (rc != TFG_OK) return rc;
+        ReadRows out;
+        out.xg = xg;
+        TFG_GUARD(return ensemble_read(h->e.device, h->e.device_index, out));
     }
     const Engine &e = h->e;
     const Geometry &g = e.geom;
@@ -792,6 +802,7 @@ int tfg_ensemble_create(tfg_ensemble **out, tfg_engine *const *engines, int n, i
             delete ens;
             return rc;
         }
+        ensemble_keep_reads(ens->dev);
         *out = ens;
     });
     return TFG_OK;
@@ -804,9 +815,9 @@ int tfg_ensemble_step(tfg_ensemble *ens, int nsteps, int use_graph) {
 
 int tfg_ensemble_destroy(tfg_ensemble *ens, int download) {
     if (!ens) return TFG_OK;
-    int rc = ensemble_destroy(ens->dev, download != 0);
+    DeviceEnsemble *dev = ens->dev;
     delete ens;
-    return rc;
+    TFG_GUARD(return ensemble_destroy(dev, download != 0));
 }
 
 double tfg_ensemble_last_ms(const tfg_ensemble *ens) {

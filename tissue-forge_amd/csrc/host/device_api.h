@@ -24,6 +24,21 @@ int ensemble_destroy(DeviceEnsemble *ens, bool download);
 // Copies the device state of every system back into its host engine.
 int ensemble_download(DeviceEnsemble *ens);
 int ensemble_download_one(DeviceEnsemble *ens, int sys);
+// Rows by particle id (null: not wanted): global positions, positions
+// relative to the cell origin, velocities (3 values each), force and number
+// density (4), species and pending flux (ns), cell ids, particle flags.
+struct ReadRows {
+    double *xg = nullptr, *x = nullptr, *v = nullptr, *f = nullptr, *sp = nullptr, *q = nullptr;
+    int *cid = nullptr, *flags = nullptr;
+    int ns = 0;
+    double origin[3] = {0, 0, 0};
+};
+// Reads system sys from the device into the caller's rows (the host engine
+// keeps its own record).
+int ensemble_read(DeviceEnsemble *ens, int sys, const ReadRows &out);
+// An ensemble whose members outlive it without a download: what was read of
+// a member is also what its host engine holds afterwards.
+void ensemble_keep_reads(DeviceEnsemble *ens);
 // Whole steps: binning, nonbonded, bonded, flux, forward Euler.
 int ensemble_step(DeviceEnsemble *ens, int nsteps, bool use_graph);
 // Binning + nonbonded + bonded force evaluation only (no update).
