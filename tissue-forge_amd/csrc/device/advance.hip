@@ -287,9 +287,9 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
         }
         return;
     }
-    // List-mode steps without bonds or angles update A in place; A is then
-    // newer than B.
-    const bool inplace = !RK4 && P.inplace != 0 && update == 1;
+    // List-mode steps update A in place (each particle reads only its own
+    // slot; the bonded terms are evaluated before); A is then newer than B.
+    const bool inplace = !RK4 && P.list_mode != 0 && update == 1;
     if (inplace && blockIdx.x == 0 && threadIdx.x == 0) P.lflags[3] = 1;
     for (int base = wstart; base < P.np; base += stride) {
         const int i = base + lane;
@@ -732,7 +732,7 @@ template <typename real> int run_energy(DeviceEnsemble *E, const KP<real> &P) {
     if (E->S > 0) {
         // the species after the update: A when the update runs in place
         hipLaunchKernelGGL(k_species_part<real>, dim3(nbx, E->nsys), dim3(256), 0, E->stream, E->d_sys,
-                           E->inplace ? P.A.sp : P.B.sp, E->np,
+                           E->list_mode ? P.A.sp : P.B.sp, E->np,
                            E->S, E->sp_part, nbx, E->d_err);
         hipLaunchKernelGGL(k_species_final, dim3(E->nsys), dim3(256), 0, E->stream, E->sp_part, nbx, E->S,
                            E->d_spec_tot, E->d_err);

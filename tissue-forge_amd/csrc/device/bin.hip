@@ -12,9 +12,8 @@
 //
 // With neighbour lists the particle order is kept between rebuilds: every
 // kernel here takes the step's rebuild flag (gate) and returns at once
-// without it, except the permute, which then copies buffer B to A in place
-// of the gather.  The cell counts are taken afresh (k_count) in the steps
-// that rebuild.
+// without it.  The cell counts are taken afresh (k_count) in the steps that
+// rebuild.
 #include <algorithm>
 
 #include "ensemble.h"
@@ -274,7 +273,7 @@ __global__ void k_sync(KP<real> P, int force) {
 }
 
 template <typename real> int run_sync(DeviceEnsemble *E, const KP<real> &P, bool force) {
-    if (!E->inplace) return TFG_OK;
+    if (!E->list_mode) return TFG_OK;
     hipLaunchKernelGGL(k_sync<real>, dim3(E->stream_grid()), dim3(E->shape.stream_threads), 0, E->stream, P,
                        force ? 1 : 0);
     return launch_error("sync");
@@ -288,28 +287,22 @@ __global__ void k_permute(KP<real> P) {
     using v4 = typename V<real>::v4;
     const int S = P.S;
     if (P.err[0] != 0) return;   // halted
-    const bool any = !P.list_mode || P.lflags[0] != 0;
-    // in-place updates: A already holds the state of systems that keep their lists
-    const bool a_current = P.inplace && P.lflags[3] != 0;
-    if (a_current && !any) return;
+    if (P.list_mode && P.lflags[0] == 0) return;   // A holds the state of systems that keep their lists
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < P.np; i += gridDim.x * blockDim.x) {
         // slot i belongs to the system of the particle buffer B holds there;
         // systems that keep their lists keep their order
-        const bool rebuild = any && (!P.list_mode || P.sflags[P.nsys + P.cell_sys[P.B.meta[i].z]] != 0);
-        if (a_current && !rebuild) continue;
-        const int src = rebuild ? P.perm[i] : i;
+        if (P.list_mode && P.sflags[P.nsys + P.cell_sys[P.B.meta[i].z]] == 0) continue;
+        const int src = P.perm[i];
         P.A.pos[i] = P.B.pos[src];
         P.A.vel[i] = P.B.vel[src];
         const int4 m = P.B.meta[src];
         P.A.meta[i] = m;
-        // A step that keeps its lists keeps every slot: the inverse mass in A
-        // and the id -> slot map are still those of the last reordering
-        if (rebuild) P.A.imass[i] = P.B.imass[src];
+        P.A.imass[i] = P.B.imass[src];
         for (int k = 0; k < S; k++) {
             P.A.sp[(size_t)k * P.np + i] = P.B.sp[(size_t)k * P.np + src];
             P.A.q[(size_t)k * P.np + i] = P.B.q[(size_t)k * P.np + src];
         }
-        if (P.list_mode && rebuild) {   // the state the new lists are built from
+        if (P.list_mode) {   // the state the new lists are built from
             v4 p = P.A.pos[i];
             P.x0[i] = p;
             P.cid0[i] = m.z;
@@ -323,7 +316,7 @@ __global__ void k_permute(KP<real> P) {
             P.A.sv[i] = P.B.sv[src];
             P.A.vk[i] = P.B.vk[src];
         }
-        if (rebuild) P.slot_of[m.y] = i;
+        P.slot_of[m.y] = i;
     }
 }
 

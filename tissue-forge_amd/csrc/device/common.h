@@ -188,9 +188,8 @@ template <typename real> struct KP {
     int coef_lds;     // 1 when every system's pair tables fit the LDS cache
     NbLayout nb;
     // Neighbour lists (null and 0 without them).
-    int list_mode;
-    int inplace;                      // list-mode steps without bonds update buffer A in place (lflags[3] set once A
-                                      // is newer than B; k_sync copies A to B where B must be current)
+    int list_mode;                    // (updates write buffer A in place)
+    int light;                        // a light step: no binning, no build, skipped while a rebuild is due
     int lcap;                         // entries per particle
     int *list;                        // entry k of particle i at list[list_index(k, i, lcap)]
     int *lcount;                      // entries per particle at the build
@@ -198,7 +197,9 @@ template <typename real> struct KP {
     typename V<real>::v4 *xb;         // position in the frame of the build cell; w: type column bits
     typename V<real>::v4 *x0;         // stored position at the build
     int *cid0;                        // cell at the build
-    int *lflags;                      // [0] some system rebuilds in this step, [2] overflow, [3] A newer than B
+    int *lflags;                      // [0] some system rebuilds in this step, [3] A newer than B (k_sync copies A to
+                                      // B where B must be current), [4] some system waits for a rebuild, [5] the
+                                      // light step in progress runs, [6] full steps that rebuilt
     int *sflags;                      // per system: [s] requested, [nsys + s] rebuilds now, [2 nsys + s] rebuilds done
     int nsys;
     int lpp, lpp_log2;                // list pass: lanes per particle (a power of two) and its log2

@@ -89,7 +89,7 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy) {
     P.coef_lds = E->coef_lds_bytes > 0 ? 1 : 0;
     P.nb = E->nb;
     P.list_mode = E->list_mode ? 1 : 0;
-    P.inplace = E->inplace ? 1 : 0;
+    P.light = 0;
     P.lpp = E->lpp;
     P.lpp_log2 = E->lpp_log2;
     P.lcap = E->lcap;
@@ -624,11 +624,6 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     E->lean_advance = deg[np] == 0 && E->S == 0;
     for (const SysDesc &d : E->sys)
         if (d.bc_active) E->lean_advance = false;
-    // List mode without bonds or angles: a step's update writes buffer A in
-    // place (each particle reads only its own slot), B is brought up to date
-    // only where it is read (a rebuilding step's binning, a force pass, a
-    // download), and steps that keep their lists skip the copy back to A.
-    E->inplace = E->list_mode && deg[np] == 0;
     {
         std::vector<int> fillp(deg.begin(), deg.end() - 1);
         // entry: kind (bit 30: angle), the particle's role in the term

@@ -53,7 +53,7 @@ template <typename real> __global__ __launch_bounds__(kReadBlock) void k_read(KP
 #pragma clang fp contract(off)
     __shared__ double lds[kReadBlock * 4];
     const SysDesc &sd = P.sys[s];
-    const bool from_a = P.inplace && P.lflags[3] != 0;   // in-place updates leave B behind A
+    const bool from_a = P.list_mode && P.lflags[3] != 0;   // in-place updates leave B behind A
     const typename V<real>::v4 *pos = from_a ? P.A.pos : P.B.pos;
     const typename V<real>::v4 *vel = from_a ? P.A.vel : P.B.vel;
     const int4 *meta = from_a ? P.A.meta : P.B.meta;
