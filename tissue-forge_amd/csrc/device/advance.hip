@@ -172,7 +172,7 @@ __device__ void reflect(const SysDesc &sd, const int loc[3], real xv[3], real vv
 // minus their sum) and its energy.  Terms out of range store zeros.
 template <typename real> __global__ __launch_bounds__(256) void k_terms(KP<real> P) {
     using v4 = typename V<real>::v4;
-    if (P.err[0] != 0) return;   // halted: the update does not read the terms
+    if (P.light ? P.lflags[5] == 0 : P.err[0] != 0) return;   // skipped or halted: the update does not read the terms
     const v4 zero = v4_of<real>(real(0), real(0), real(0));
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < P.nbonds + P.nangles; t += gridDim.x * blockDim.x) {
         if (t < P.nbonds) {
@@ -268,6 +268,10 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
     const int lane = threadIdx.x & 63;
     const int wstart = (blockIdx.x * blockDim.x + threadIdx.x) - lane;
     const int stride = gridDim.x * blockDim.x;
+    if (P.light) {   // the step's counter moves here, where nothing reads it
+        if (P.lflags[5] == 0) return;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *P.step += 1;
+    }
     // Halted (the update writes its own failure to err[1], not to this word).
     const int halt = P.err[0];
     if (halt & kHaltTooFast) return;
@@ -585,7 +589,10 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
                 const int leader = __builtin_ctzll(req);
                 const int s = __shfl(sysid, leader);
                 req &= ~__ballot(sysid == s);
-                if (lane == leader && P.sflags[s] == 0) atomicOr(&P.sflags[s], 1);
+                if (lane == leader && P.sflags[s] == 0) {
+                    atomicOr(&P.sflags[s], 1);
+                    P.lflags[4] = 1;
+                }
             }
             continue;   // the counts are taken afresh when the lists are rebuilt
         }

@@ -121,6 +121,18 @@ struct DeviceEnsemble {
     long long *d_step = nullptr;
     int *d_err = nullptr;
 
+    // What the host needs to know after a call, written by k_report into
+    // pinned memory as the call's last kernel; then each system's 5 sums.
+    struct Status {
+        long long step;
+        int err[2];
+        int due;        // some system waits for a rebuild
+        int rebuilds;   // full steps that rebuilt
+    };
+    Status *status = nullptr;
+    double *status_sums() const { return reinterpret_cast<double *>(status + 1); }
+    int light_run = 4;   // light steps between two full ones
+
     // Readback: a pinned buffer and an event per reading thread.
     struct ReadSlot {
         unsigned char *ptr = nullptr;
@@ -137,6 +149,7 @@ struct DeviceEnsemble {
     std::vector<char> kept_sys;
 
     ~DeviceEnsemble() {
+        if (status) (void)hipHostFree(status);
         for (ReadSlot &r : read_slot) {
             if (r.ptr) (void)hipHostFree(r.ptr);
             if (r.done) (void)hipEventDestroy(r.done);

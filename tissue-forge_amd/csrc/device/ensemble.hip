@@ -120,6 +120,7 @@ __global__ void k_tick(long long *step, int *err) {
 // it (or its state was just uploaded or rebinned); the requests are
 // consumed.  lflags[0] tells the binning kernels that some system rebuilds.
 __global__ __launch_bounds__(256) void k_tick_list(long long *step, int *lflags, int *sflags, int nsys, int *err) {
+    // (a full step answers every request there is: lflags[4] starts anew)
     __shared__ int any, halted;
     if (threadIdx.x == 0) {
         halted = tick_halted(err) ? 1 : 0;
@@ -138,13 +139,46 @@ __global__ __launch_bounds__(256) void k_tick_list(long long *step, int *lflags,
     }
     if (mine) atomicOr(&any, 1);
     __syncthreads();
-    if (threadIdx.x == 0) lflags[0] = any;
+    if (threadIdx.x == 0) {
+        lflags[0] = any;
+        lflags[4] = 0;
+        lflags[6] += any;
+    }
+}
+
+// The call's outcome for the host (DeviceEnsemble::Status), and the energies.
+__global__ __launch_bounds__(256) void k_report(const long long *step, const int *err, const int *lflags,
+                                                const double *energy, int n, DeviceEnsemble::Status *out) {
+    if (threadIdx.x == 0) {
+        out->step = *step;
+        out->err[0] = err[0];
+        out->err[1] = err[1];
+        out->due = lflags[4];
+        out->rebuilds = lflags[6];
+    }
+    double *sums = reinterpret_cast<double *>(out + 1);
+    for (int k = threadIdx.x; k < n; k += blockDim.x) sums[k] = energy[k];
+}
+
+static int report(DeviceEnsemble *E) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(256), 0, E->stream, E->d_step, E->d_err, E->d_lflags, E->d_energy,
+                       5 * E->nsys, E->status);
+    return launch_error("report");
+}
+
+// The end of a step call: its device time ends, the report, and the wait.
+static int finish(DeviceEnsemble *E) {
+    TFG_HIP(hipEventRecord(E->ev[6], E->stream));
+    const int rc = report(E);
+    if (rc != TFG_OK) return rc;
+    TFG_HIP(hipStreamSynchronize(E->stream));
+    return TFG_OK;
 }
 
 // A force pass outside a step rebins every system and leaves the next step
 // a rebuild to do, since the order changed under the lists.
 __global__ __launch_bounds__(256) void k_list_rebin(int *lflags, int *sflags, int nsys) {
-    if (threadIdx.x == 0) lflags[0] = 1;
+    if (threadIdx.x == 0) lflags[0] = lflags[4] = 1;
     for (int s = threadIdx.x; s < nsys; s += blockDim.x) {
         sflags[s] = 1;
         sflags[nsys + s] = 1;
@@ -283,9 +317,9 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         for (int k = 0; k < 8; k++) TFG_HIP(hipEventCreate(&E->ev[k]));
         E->nev = 8;
     }
-    hipDeviceProp_t prop;
-    TFG_HIP(hipGetDeviceProperties(&prop, E->device));
-    E->cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+    int cus = 0;
+    TFG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, E->device));
+    E->cus = cus > 0 ? cus : 256;
     const int nsys = static_cast<int>(E->engines.size());
     E->nsys = nsys;
     // FP32 positions are stored relative to the cell centre.
@@ -696,7 +730,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     E->nbonds = static_cast<int>(hb.size());
     E->nangles = static_cast<int>(ha.size());
     ALLOC(E->d_tforce, v4, hb.size() + 2 * ha.size());
-    ALLOC(E->d_lflags, int, 4);
+    ALLOC(E->d_lflags, int, 8);
     ALLOC(E->d_sflags, int, 3 * nsys);
     if (E->list_mode) {
         // slack for the list pass, which reads up to 8 batches of 4 entries
@@ -744,7 +778,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         if ((rc = H2D(static_cast<v4 *>(E->xb) + np, &far, sizeof(v4)))) return rc;
     }
     {
-        const int flags[4] = {0, 0, 0, 0};
+        const int flags[8] = {0, 0, 0, 0, 1, 0, 0, 0};   // [4]: the first step builds
         if ((rc = H2D(E->d_lflags, flags, sizeof(flags)))) return rc;
         std::vector<int> sfl(3 * nsys, 0);
         for (int s = 0; s < nsys; s++) sfl[s] = 1;   // the first step builds every system's lists
@@ -760,6 +794,14 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         TFG_HIP(hipMemset(p, 0, sizeof(double) * (size_t)np));
     TFG_HIP(hipMemset(E->d_energy, 0, sizeof(double) * 5 * nsys));
     TFG_HIP(hipMemset(E->d_spec_tot, 0, sizeof(double) * kMaxSpecies * nsys));
+    if (!E->no_alloc) {
+        void *p = nullptr;
+        const size_t bytes = sizeof(DeviceEnsemble::Status) + sizeof(double) * 5 * nsys;
+        TFG_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+        std::memset(p, 0, bytes);
+        E->status = static_cast<DeviceEnsemble::Status *>(p);
+        E->status->due = 1;
+    }
     TFG_HIP(hipDeviceSynchronize());
     // (list mode counts the cells when it rebuilds)
     if (!E->list_mode && (rc = run_count(E)) != TFG_OK) return rc;
@@ -798,29 +840,83 @@ int ensemble_download(DeviceEnsemble *E) { return download(E, -1); }
 
 int ensemble_download_one(DeviceEnsemble *E, int sys) { return download(E, sys); }
 
+// One energy-free full step as a graph, captured on first use.
+template <typename real> static int step_graph(DeviceEnsemble *E) {
+    if (E->graph) return TFG_OK;
+    TFG_HIP(hipStreamBeginCapture(E->stream, hipStreamCaptureModeThreadLocal));
+    const int rc = enqueue_step<real>(E, false, nullptr);
+    hipGraph_t captured = nullptr;
+    const hipError_t ce = hipStreamEndCapture(E->stream, &captured);
+    if (rc != TFG_OK) {
+        if (captured) (void)hipGraphDestroy(captured);
+        return rc;
+    }
+    if (ce != hipSuccess) return set_error(TFG_E_DEVICE, std::string("graph capture: ") + hipGetErrorString(ce));
+    const hipError_t ie = hipGraphInstantiate(&E->graph, captured, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(captured);
+    if (ie != hipSuccess) return set_error(TFG_E_DEVICE, std::string("graph instantiate: ") + hipGetErrorString(ie));
+    return TFG_OK;
+}
+
+// nsteps list-mode steps, the last one with energies.
+//
+// Only the steps that rebuild need the binning and the build, but whether a
+// step rebuilds is decided on the device, and a full step that keeps its
+// lists still launches the whole chain: nine kernels that return at once, 17
+// us of the 43 us step of 8,000 FP64 particles.  So most steps are light (pair
+// pass, terms, update); a light step finds out by itself that a rebuild is
+// due and then does nothing, until the next full step answers.  The steps
+// come out the same, whichever slot runs them.  A run of light steps between
+// full ones costs the chain once per run, and each rebuild wastes half a run
+// of launches that do nothing: with ~17 us and ~4 us that is least at
+// sqrt(8 x the steps from one rebuild to the next).  Every slot runs one step
+// at most, so the call sends as many slots as steps are left, looks at the
+// counter, and sends the rest.
+template <typename real> static int list_steps(DeviceEnsemble *E, int nsteps) {
+    int rc;
+    KP<real> L = make_params<real>(E, 0);
+    L.light = 1;
+    L.step_ahead = 1;   // the update counts the step, after the pair pass
+    for (int left = nsteps; left > 0;) {
+        const DeviceEnsemble::Status before = *E->status;
+        bool full = before.due != 0;
+        for (int k = 0, run = 0; k < left - 1; k++) {
+            if (full || run >= E->light_run) {
+                if ((rc = step_graph<real>(E)) != TFG_OK) return rc;
+                TFG_HIP(hipGraphLaunch(E->graph, E->stream));
+                full = false;
+                run = 0;
+                continue;
+            }
+            if ((rc = run_list_force<real>(E, L)) != TFG_OK || (rc = run_advance<real>(E, L, 1)) != TFG_OK) return rc;
+            run++;
+        }
+        if ((rc = enqueue_step<real>(E, true, nullptr)) != TFG_OK || (rc = finish(E)) != TFG_OK) return rc;
+        const DeviceEnsemble::Status &now = *E->status;
+        if (now.err[0] != 0 || now.err[1] != 0) break;
+        const int done = static_cast<int>(now.step - before.step), built = now.rebuilds - before.rebuilds;
+        if (done < 1 || done > left) return set_error(TFG_E_DEVICE, "list steps: the step counter is off");
+        left -= done;
+        if (built > 0)
+            E->light_run = std::max(1, std::min(32, static_cast<int>(std::sqrt(8.0 * done / built))));
+        else if (done > E->light_run)
+            E->light_run = std::min(32, 2 * E->light_run);
+    }
+    return TFG_OK;
+}
+
 template <typename real> static int step_t(DeviceEnsemble *E, int nsteps, bool use_graph) {
     int rc;
     constexpr int kEv = 5;   // phase events per step
     TFG_HIP(hipEventRecord(E->ev[5], E->stream));
-    if (use_graph && nsteps > 1 && !E->profile) {
+    if (use_graph && nsteps > 1 && !E->profile && E->list_mode && E->nr_fluxsteps == 1) {
+        if ((rc = list_steps<real>(E, nsteps)) != TFG_OK) return rc;
+    } else if (use_graph && nsteps > 1 && !E->profile) {
         // One energy-free step is captured once and replayed; the last step
         // runs eagerly with the energy pass.
-        if (!E->graph) {
-            TFG_HIP(hipStreamBeginCapture(E->stream, hipStreamCaptureModeThreadLocal));
-            rc = enqueue_step<real>(E, false, nullptr);
-            hipGraph_t captured = nullptr;
-            hipError_t ce = hipStreamEndCapture(E->stream, &captured);
-            if (rc != TFG_OK) {
-                if (captured) (void)hipGraphDestroy(captured);
-                return rc;
-            }
-            if (ce != hipSuccess) return set_error(TFG_E_DEVICE, std::string("graph capture: ") + hipGetErrorString(ce));
-            hipError_t ie = hipGraphInstantiate(&E->graph, captured, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(captured);
-            if (ie != hipSuccess) return set_error(TFG_E_DEVICE, std::string("graph instantiate: ") + hipGetErrorString(ie));
-        }
+        if ((rc = step_graph<real>(E)) != TFG_OK) return rc;
         for (int k = 0; k < nsteps - 1; k++) TFG_HIP(hipGraphLaunch(E->graph, E->stream));
-        if ((rc = enqueue_step<real>(E, true, nullptr)) != TFG_OK) return rc;
+        if ((rc = enqueue_step<real>(E, true, nullptr)) != TFG_OK || (rc = finish(E)) != TFG_OK) return rc;
     } else {
         if (E->profile && static_cast<int>(E->prof_ev.size()) < kEv * nsteps) {
             for (size_t k = E->prof_ev.size(); k < static_cast<size_t>(kEv * nsteps); k++) {
@@ -833,9 +929,8 @@ template <typename real> static int step_t(DeviceEnsemble *E, int nsteps, bool u
             hipEvent_t *ev = E->profile ? &E->prof_ev[kEv * k] : (k == nsteps - 1 ? E->ev : nullptr);
             if ((rc = enqueue_step<real>(E, k == nsteps - 1, ev)) != TFG_OK) return rc;
         }
+        if ((rc = finish(E)) != TFG_OK) return rc;
     }
-    TFG_HIP(hipEventRecord(E->ev[6], E->stream));
-    TFG_HIP(hipStreamSynchronize(E->stream));
     TFG_HIP(hipEventElapsedTime(&E->last_ms, E->ev[5], E->ev[6]));
     if (!use_graph || nsteps <= 1 || E->profile) {
         hipEvent_t *last = E->profile ? &E->prof_ev[kEv * (nsteps - 1)] : E->ev;
@@ -862,14 +957,15 @@ template <typename real> static int step_t(DeviceEnsemble *E, int nsteps, bool u
     // for a particle moving too fast, before the pair pass for a list
     // overflow, as the reference's engine_step returns after time += 1
     // (tfEngine.cpp:1388-1402, tf_engine_advance.cpp:482-489).
-    int err[2] = {0, 0};
-    TFG_HIP(hipMemcpy(err, E->d_err, sizeof(err), hipMemcpyDeviceToHost));
+    int err[2] = {E->status->err[0], E->status->err[1]};
     if (err[1]) err[0] |= kHaltTooFast;
     if (err[0]) {
         TFG_HIP(hipMemset(E->d_err, 0, sizeof(err)));
         if (E->list_mode) {   // every system rebuilds at the next step
             std::vector<int> req(E->nsys, 1);
             TFG_HIP(hipMemcpy(E->d_sflags, req.data(), sizeof(int) * E->nsys, hipMemcpyHostToDevice));
+            TFG_HIP(hipMemcpy(E->d_lflags + 4, req.data(), sizeof(int), hipMemcpyHostToDevice));
+            E->status->due = 1;
         }
         if (err[0] & kHaltTooFast)
             return set_error(TFG_E_TOOFAST, "particle moving too fast (moved two cells or more in one step)");
@@ -881,11 +977,8 @@ template <typename real> static int step_t(DeviceEnsemble *E, int nsteps, bool u
 
 // Step counter of every system from the device (engine->time): the steps
 // begun since the upload, a failing one included.
-static int sync_time(DeviceEnsemble *E) {
-    long long steps = 0;
-    TFG_HIP(hipMemcpy(&steps, E->d_step, sizeof(steps), hipMemcpyDeviceToHost));
-    for (int s = 0; s < E->nsys; s++) E->engines[s]->time = E->sys[s].time0 + steps;
-    return TFG_OK;
+static void sync_time(DeviceEnsemble *E) {
+    for (int s = 0; s < E->nsys; s++) E->engines[s]->time = E->sys[s].time0 + E->status->step;
 }
 
 int ensemble_list_entries(DeviceEnsemble *E, int sys, double *mean, int *maxn) {
@@ -929,8 +1022,7 @@ int ensemble_step(DeviceEnsemble *E, int nsteps, bool use_graph) {
     if (rc == TFG_E_DEVICE) return rc;
     // also after a failed step: the host time counts the steps begun
     const std::string msg = rc != TFG_OK ? std::string(last_error()) : std::string();
-    const int rt = sync_time(E);
-    if (rt != TFG_OK) return rt;
+    sync_time(E);
     return rc != TFG_OK ? set_error(rc, msg) : TFG_OK;
 }
 
@@ -956,6 +1048,7 @@ template <typename real> static int force_t(DeviceEnsemble *E) {
     if ((rc = run_advance<real>(E, P, 0)) != TFG_OK) return rc;
     if (timed) TFG_HIP(hipEventRecord(E->ev[4], E->stream));
     if ((rc = run_energy<real>(E, P)) != TFG_OK) return rc;
+    if (E->status && (rc = report(E)) != TFG_OK) return rc;
     TFG_HIP(hipStreamSynchronize(E->stream));
     for (int k = 0; k < 4 && timed; k++) {
         float ms = 0;
@@ -1014,6 +1107,10 @@ int ensemble_force(DeviceEnsemble *E) {
 
 int ensemble_energies(DeviceEnsemble *E, int s, Energies *out) {
     if (s < 0 || s >= E->nsys) return set_error(TFG_E_RANGE, "system index out of range");
+    if (E->status) {   // every call that evaluates them ends with a report
+        *out = energies_of(E->status_sums() + 5 * s);
+        return TFG_OK;
+    }
     double e[5];
     TFG_HIP(hipStreamSynchronize(E->stream));
     TFG_HIP(hipMemcpy(e, E->d_energy + 5 * s, sizeof(e), hipMemcpyDeviceToHost));

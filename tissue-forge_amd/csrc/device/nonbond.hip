@@ -1164,7 +1164,16 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ FluxDesc<real> s_flux[FLUX ? kMaxFluxEntries : 1];
     __shared__ int2 s_fmap[FLUX ? kMaxTypes * kMaxTypes : 1];
-    if (P.err[0] != 0) return;   // halted (nothing writes the word during this kernel)
+    if (P.light) {
+        // A light step runs unless the ensemble is halted or a system waits
+        // for its rebuild; nothing writes these words during this kernel, and
+        // the kernels after it take the decision from lflags[5].
+        const bool go = P.err[0] == 0 && P.err[1] == 0 && P.lflags[4] == 0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) P.lflags[5] = go ? 1 : 0;
+        if (!go) return;
+    } else if (P.err[0] != 0) {
+        return;   // halted (nothing writes the word during this kernel)
+    }
     // Workgroups go to the 8 XCDs in turn: the workgroups of one XCD take
     // consecutive particle blocks (the grid is a multiple of 8), so that the
     // partner positions they gather meet in that XCD's L2.
