@@ -298,14 +298,15 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
     for (int base = wstart; base < P.np; base += stride) {
         const int i = base + lane;
         const bool valid = i < P.np;
-        int newc = -1;
-        bool far_moved = false;
+        int newc = -1, sysid = -1;
+        bool far_moved = false, near_moved = false, near_retry = false;
         if (valid) {
             const int4 mi = P.A.meta[i];
             const int c = mi.z;
             const int id = mi.y;
             const int info = mi.x;
-            const SysDesc &sd = P.sys[P.cell_sys[c]];
+            sysid = P.cell_sys[c];
+            const SysDesc &sd = P.sys[sysid];
             v4 p = P.A.pos[i];
             v4 v = P.A.vel[i];
             v4 f = P.force[i];
@@ -558,6 +559,21 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
                 b.y = xbv[1];
                 b.z = xbv[2];
                 b.w = as_real_bits(type_column<v4>(info & 0xffff), real(0));
+                const int mode = P.sflags[3 * P.nsys + sysid];
+                if (mode != kListAll) {
+                    // the displacement since the near lists were made
+                    v4 q;
+                    if (mode == kListMakeNear && !P.light) {   // in this step's pair pass
+                        q = P.xb[i];
+                        P.xn[i] = q;
+                    } else {
+                        q = P.xn[i];
+                    }
+                    const real nx = xbv[0] - q.x, ny = xbv[1] - q.y, nz = xbv[2] - q.z;
+                    near_moved = nx * nx + ny * ny + nz * nz > real(sd.near_half2);
+                } else {
+                    near_retry = i == sd.p_off && P.lflags[7] + 1 - P.sflags[5 * P.nsys + sysid] >= P.sflags[6 * P.nsys + sysid];
+                }
                 P.xb[i] = b;
             }
             // Particles that changed cell skip this step's integration and keep
@@ -582,8 +598,7 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
         }
         if (P.list_mode) {
             // One request per system present in the wave, and none once its
-            // flag is up.
-            const int sysid = valid ? P.cell_sys[newc] : -1;
+            // flag is up: a rebuild, or new near lists.
             unsigned long long req = __ballot(far_moved);
             while (req != 0ull) {
                 const int leader = __builtin_ctzll(req);
@@ -594,6 +609,17 @@ __global__ __launch_bounds__(256) void k_advance(KP<real> P, int update) {
                     P.lflags[4] = 1;
                 }
             }
+            req = __ballot(near_moved);
+            while (req != 0ull) {
+                const int leader = __builtin_ctzll(req);
+                const int s = __shfl(sysid, leader);
+                req &= ~__ballot(sysid == s);
+                if (lane == leader && P.sflags[4 * P.nsys + s] == 0) {
+                    atomicOr(&P.sflags[4 * P.nsys + s], 1);
+                    P.lflags[4] = 1;
+                }
+            }
+            if (near_retry) P.lflags[4] = 1;
             continue;   // the counts are taken afresh when the lists are rebuilt
         }
         int head, len;

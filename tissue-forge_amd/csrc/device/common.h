@@ -64,6 +64,9 @@ struct SysDesc {
     int nstencil_b, stencil_off_b, span_z_b;
     double cutb2;        // (cutoff + skin)^2, widened by a relative 1e-5
     double skin_half2;   // (skin / 2)^2, narrowed by a relative 1e-4
+    // Near lists: the list entries within cutoff + near skin, kept until a
+    // particle has moved by half the near skin (the same margins).
+    double cutn2, near_half2;
 };
 
 // Halt bits of the device error word (KP::err[0]).
@@ -80,14 +83,26 @@ constexpr int kCentreCode = 62;        // list_code(0, 0, 0)
 // each list to a multiple of it with entries naming the slot np, a dummy
 // record far from every particle (its pair is outside any cutoff).
 constexpr int kListBatch = 4;
+// List mode of a system in a step: the pair pass reads the lists as built,
+// the near lists, or near lists made in this step.
+constexpr int kListAll = 0, kListNear = 1, kListMakeNear = 2;
+// Near lists that served fewer than kNearLife steps cost more than they save:
+// the system then reads the whole lists for kNearRetry steps from their making,
+// twice as long after each such try, up to kNearRetryMost.
+constexpr int kNearLife = 4, kNearRetry = 16, kNearRetryMost = 256;
+constexpr int kNearMostCap = 65535;   // entries per particle (ncount's fields)
+constexpr int kNearShare = 8;   // age from which near lists are renewed with another system's
 constexpr float kListFar = 1.0e6f;
 constexpr int kMaxBuildCells = 128;    // build stencil cells (at most 5^3)
-// Entry k of particle i: tiles of 64 particles, entry-major inside a tile, so
-// that a wave of consecutive particles reads one entry index as 256
-// contiguous bytes and one tile's entries stay within lcap * 256 bytes.
-__host__ __device__ inline size_t list_index(int k, int i, int lcap) {
-    return (static_cast<size_t>(i >> 6) * lcap + k) * 64 + (i & 63);
+// Entry k of particle i: tiles of 64 particles of lcap * 256 bytes, inside a
+// tile batch by batch and a batch's particles in turn, so that a lane reads
+// a batch of its particle as one 16-byte load and a wave of consecutive
+// particles reads 1 KB in a row.  list_base is a particle's first entry,
+// list_row the distance of entry k from it.
+__host__ __device__ inline size_t list_base(int i, int lcap) {
+    return static_cast<size_t>(i >> 6) * lcap * 64 + (i & 63) * kListBatch;
 }
+__host__ __device__ inline int list_row(int k) { return (k & ~(kListBatch - 1)) * 64 + (k & (kListBatch - 1)); }
 // Pair descriptors in LDS: kPairVecs fields, each an array of kDescPairs
 // vectors (one per type pair, ti * ntypes + tj), so that lanes reading the
 // descriptors of different type pairs spread over the LDS banks.  A particle
@@ -191,16 +206,25 @@ template <typename real> struct KP {
     int list_mode;                    // (updates write buffer A in place)
     int light;                        // a light step: no binning, no build, skipped while a rebuild is due
     int lcap;                         // entries per particle
-    int *list;                        // entry k of particle i at list[list_index(k, i, lcap)]
+    int *list;                        // entry k of particle i at list[list_base(i, lcap) + list_row(k)]
     int *lcount;                      // entries per particle at the build
-    const int4 *lblock;               // list kernel blocks: system, first slot, count
+    int *ncount;                      // near lists (a list's entries within reach of the near skin, in list order):
+                                      // entries, and << 16 the batch of the particle's tile rows they start at,
+                                      // behind the lists
+    typename V<real>::v4 *xn;         // position in the build cell's frame when the near lists were made
+    const int4 *lblock;               // list kernel chunks: system, first slot, count
+    const unsigned char *limage;      // per system, nb.total bytes: the pair pass's LDS contents (k_list_image)
     typename V<real>::v4 *xb;         // position in the frame of the build cell; w: type column bits
     typename V<real>::v4 *x0;         // stored position at the build
     int *cid0;                        // cell at the build
     int *lflags;                      // [0] some system rebuilds in this step, [3] A newer than B (k_sync copies A to
-                                      // B where B must be current), [4] some system waits for a rebuild, [5] the
-                                      // light step in progress runs, [6] full steps that rebuilt
-    int *sflags;                      // per system: [s] requested, [nsys + s] rebuilds now, [2 nsys + s] rebuilds done
+                                      // B where B must be current), [4] some system waits for a full step, [5] the
+                                      // light step in progress runs, [6] full steps that were waited for, [7] the
+                                      // number of the step in progress (low bits)
+    int *sflags;                      // per system: [s] requested, [nsys + s] rebuilds now, [2 nsys + s] rebuilds done,
+                                      // [3 nsys + s] list mode (kListAll ..), [4 nsys + s] near lists outlived,
+                                      // [5 nsys + s] step of the last near lists (low bits), [6 nsys + s] steps from
+                                      // one try of them to the next
     int nsys;
     int lpp, lpp_log2;                // list pass: lanes per particle (a power of two) and its log2
 };

@@ -80,8 +80,10 @@ struct DeviceEnsemble {
     int lpp = 1, lpp_log2 = 0;  // list pass lanes per particle
     int nlblocks = 0;
     int4 *d_lblock = nullptr;
+    unsigned char *d_limage = nullptr;
     int *d_list = nullptr, *d_lcount = nullptr, *d_cid0 = nullptr, *d_lflags = nullptr, *d_sflags = nullptr;
-    void *xb = nullptr, *x0 = nullptr;
+    int *d_ncount = nullptr;
+    void *xb = nullptr, *x0 = nullptr, *xn = nullptr;
     int nonbond_resident = 0; // pair-kernel workgroups resident on the device at once
     LaunchShape shape;
     Buffers buf;
@@ -126,8 +128,8 @@ struct DeviceEnsemble {
     struct Status {
         long long step;
         int err[2];
-        int due;        // some system waits for a rebuild
-        int rebuilds;   // full steps that rebuilt
+        int due;      // some system waits for a full step
+        int served;   // full steps that were waited for
     };
     Status *status = nullptr;
     double *status_sums() const { return reinterpret_cast<double *>(status + 1); }
@@ -206,6 +208,9 @@ template <typename real> int run_advance(DeviceEnsemble *E, const KP<real> &P, i
 // Neighbour lists: the build (a variant of the pair kernel over the wider
 // stencil, run when the step rebuilds) and the list pair kernel.
 template <typename real> int run_list_build(DeviceEnsemble *E, const KP<real> &P);
+// The pair pass's LDS contents of every system, once after the upload.
+template <typename real> int run_list_image(DeviceEnsemble *E, const KP<real> &P);
+template <typename real> int run_near(DeviceEnsemble *E, const KP<real> &P);
 template <typename real> int run_list_force(DeviceEnsemble *E, const KP<real> &P);
 // The flux-only list pass of a flux sub-step (pending flux, no forces).
 template <typename real> int run_list_flux(DeviceEnsemble *E, const KP<real> &P);

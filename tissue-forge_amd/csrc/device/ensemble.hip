@@ -95,7 +95,10 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy) {
     P.lcap = E->lcap;
     P.list = E->d_list;
     P.lcount = E->d_lcount;
+    P.ncount = E->d_ncount;
+    P.xn = static_cast<v4 *>(E->xn);
     P.lblock = E->d_lblock;
+    P.limage = E->d_limage;
     P.xb = static_cast<v4 *>(E->xb);
     P.x0 = static_cast<v4 *>(E->x0);
     P.cid0 = E->d_cid0;
@@ -119,12 +122,26 @@ __global__ void k_tick(long long *step, int *err) {
 // List mode: a system rebuilds in this step when the last advance asked for
 // it (or its state was just uploaded or rebinned); the requests are
 // consumed.  lflags[0] tells the binning kernels that some system rebuilds.
+//
+// Near lists.  The lists reach cutoff + skin, so that rebuilds are rare, but
+// every step pays for the entries beyond the cutoff: 42% of them at skin 0.2
+// cutoffs.  The pair pass is bound by its entries, so it reads near lists:
+// those entries within cutoff + a third of the skin (k_near), good until a
+// particle has moved by half that.  Step calls with a quarter, a third, 0.4
+// and a half of the skin: 2M mixture 21.1, 20.5, 22.0, 22.2 ms (26.8 without
+// near lists), 1M chains 8.1, 7.8, 7.9, 8.0 (8.3), 8k FP64 2.42, 2.38, 2.35,
+// 2.34 (2.47).  Where particles outrun them (DPD droplets in their first
+// steps) the system goes back to the whole lists, for longer each time.
+// Which list a step reads follows from the steps before it alone, never from
+// how the host groups steps into calls: whatever changes it raises lflags[4],
+// so that the next step is a full one.
 __global__ __launch_bounds__(256) void k_tick_list(long long *step, int *lflags, int *sflags, int nsys, int *err) {
     // (a full step answers every request there is: lflags[4] starts anew)
-    __shared__ int any, halted;
+    __shared__ int any, halted, now;
     if (threadIdx.x == 0) {
         halted = tick_halted(err) ? 1 : 0;
         if (!halted) *step += 1;
+        now = static_cast<int>(*step);
         any = 0;
     }
     __syncthreads();
@@ -136,13 +153,32 @@ __global__ __launch_bounds__(256) void k_tick_list(long long *step, int *lflags,
         sflags[nsys + s] = rb;
         sflags[2 * nsys + s] += rb;
         mine |= rb;
+        const bool had = sflags[3 * nsys + s] != kListAll;
+        const int age = now - sflags[5 * nsys + s];
+        // In an ensemble one system that is waited for renews the near lists
+        // of some age with it: with each at its own time every step of 48
+        // replicas was a full one (20 steps 4.7 ms, together 4.0).
+        const bool lost = rb != 0 || sflags[4 * nsys + s] != 0 || (lflags[4] != 0 && age >= kNearShare);
+        sflags[4 * nsys + s] = 0;
+        int mode = had ? kListNear : kListAll;
+        if (had && lost) {
+            int &wait = sflags[6 * nsys + s];
+            const bool paid = age >= kNearLife;
+            wait = paid ? kNearRetry : min(2 * wait, kNearRetryMost);
+            mode = paid ? kListMakeNear : kListAll;
+        } else if (!had && age >= sflags[6 * nsys + s]) {
+            mode = kListMakeNear;
+        }
+        if (mode == kListMakeNear) sflags[5 * nsys + s] = now;
+        sflags[3 * nsys + s] = mode;
     }
     if (mine) atomicOr(&any, 1);
     __syncthreads();
     if (threadIdx.x == 0) {
         lflags[0] = any;
+        lflags[6] += lflags[4];
         lflags[4] = 0;
-        lflags[6] += any;
+        lflags[7] = now;
     }
 }
 
@@ -154,7 +190,7 @@ __global__ __launch_bounds__(256) void k_report(const long long *step, const int
         out->err[0] = err[0];
         out->err[1] = err[1];
         out->due = lflags[4];
-        out->rebuilds = lflags[6];
+        out->served = lflags[6];
     }
     double *sums = reinterpret_cast<double *>(out + 1);
     for (int k = threadIdx.x; k < n; k += blockDim.x) sums[k] = energy[k];
@@ -205,7 +241,7 @@ template <typename real> static int enqueue_step(DeviceEnsemble *E, bool energy,
         if (ev) TFG_HIP(hipEventRecord(ev[0], E->stream));
         if ((rc = run_bin<real>(E, Pe)) != TFG_OK) return rc;
         if (ev) TFG_HIP(hipEventRecord(ev[1], E->stream));
-        if ((rc = run_list_build<real>(E, Pe)) != TFG_OK) return rc;
+        if ((rc = run_list_build<real>(E, Pe)) != TFG_OK || (rc = run_near<real>(E, Pe)) != TFG_OK) return rc;
         if (ev) TFG_HIP(hipEventRecord(ev[2], E->stream));
         // flux sub-steps (tf_engine_advance.cpp:313-323): the flux-only list
         // pass, then Fluxes_integrate, nr_fluxsteps - 1 times
@@ -413,6 +449,9 @@ template <typename real> static int upload(DeviceEnsemble *E) {
             d.cutb2 = rcs * rcs * (1.0 + 1e-5);
             const double half = 0.5 * e.verlet_skin * (1.0 - 1e-4);
             d.skin_half2 = half * half;
+            const double near = e.verlet_skin / 3.0, near_half = 0.5 * near * (1.0 - 1e-4);
+            d.cutn2 = (e.geom.cutoff + near) * (e.geom.cutoff + near) * (1.0 + 1e-5);
+            d.near_half2 = near_half * near_half;
             double vol = 1.0;
             for (int k = 0; k < 3; k++) vol *= e.geom.cdim[k] * e.geom.h[k];   // the volume the cell grid spans
             const double expect = (vol > 0 ? e.parts.size() / vol : 0.0) * 4.0 / 3.0 * M_PI * rcs * rcs * rcs;
@@ -731,14 +770,17 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     E->nangles = static_cast<int>(ha.size());
     ALLOC(E->d_tforce, v4, hb.size() + 2 * ha.size());
     ALLOC(E->d_lflags, int, 8);
-    ALLOC(E->d_sflags, int, 3 * nsys);
+    ALLOC(E->d_sflags, int, 7 * nsys);
     if (E->list_mode) {
         // slack for the list pass, which reads up to 8 batches of 4 entries
         // past a list's end
         ALLOC(E->d_list, int, (size_t)((np + 63) / 64) * 64 * E->lcap + 64 * 64);
         ALLOC(E->d_lcount, int, np);
+        ALLOC(E->d_ncount, int, np);
+        ALLOC(E->xn, v4, np);
         ALLOC(E->d_cid0, int, np);
         ALLOC(E->d_lblock, int4, lblocks.size());
+        ALLOC(E->d_limage, unsigned char, static_cast<size_t>(nsys) * E->nbl.total);
         ALLOC(E->xb, v4, np + 1);   // slot np: the dummy that pads the lists
         ALLOC(E->x0, v4, np);
     }
@@ -780,8 +822,12 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     {
         const int flags[8] = {0, 0, 0, 0, 1, 0, 0, 0};   // [4]: the first step builds
         if ((rc = H2D(E->d_lflags, flags, sizeof(flags)))) return rc;
-        std::vector<int> sfl(3 * nsys, 0);
-        for (int s = 0; s < nsys; s++) sfl[s] = 1;   // the first step builds every system's lists
+        std::vector<int> sfl(7 * nsys, 0);
+        for (int s = 0; s < nsys; s++) {
+            sfl[s] = 1;   // the first step builds every system's lists, and its near lists
+            sfl[5 * nsys + s] = -kNearRetry;
+            sfl[6 * nsys + s] = E->lcap <= kNearMostCap ? kNearRetry : 0x7fffffff;   // (never)
+        }
         if ((rc = H2D(E->d_sflags, sfl.data(), sizeof(int) * sfl.size()))) return rc;
     }
     // Zeroed state (outside any graph capture).
@@ -803,6 +849,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         E->status->due = 1;
     }
     TFG_HIP(hipDeviceSynchronize());
+    if (E->list_mode && (rc = run_list_image<real>(E, make_params<real>(E, 0))) != TFG_OK) return rc;
     // (list mode counts the cells when it rebuilds)
     if (!E->list_mode && (rc = run_count(E)) != TFG_OK) return rc;
     TFG_HIP(hipStreamSynchronize(E->stream));
@@ -864,12 +911,13 @@ template <typename real> static int step_graph(DeviceEnsemble *E) {
 // step rebuilds is decided on the device, and a full step that keeps its
 // lists still launches the whole chain: nine kernels that return at once, 17
 // us of the 43 us step of 8,000 FP64 particles.  So most steps are light (pair
-// pass, terms, update); a light step finds out by itself that a rebuild is
-// due and then does nothing, until the next full step answers.  The steps
+// pass, terms, update); a light step finds out by itself that a rebuild (or
+// new near lists) is due and then does nothing, until the next full step
+// answers.  The steps
 // come out the same, whichever slot runs them.  A run of light steps between
 // full ones costs the chain once per run, and each rebuild wastes half a run
 // of launches that do nothing: with ~17 us and ~4 us that is least at
-// sqrt(8 x the steps from one rebuild to the next).  Every slot runs one step
+// sqrt(8 x the steps from one wait to the next).  Every slot runs one step
 // at most, so the call sends as many slots as steps are left, looks at the
 // counter, and sends the rest.
 template <typename real> static int list_steps(DeviceEnsemble *E, int nsteps) {
@@ -894,11 +942,11 @@ template <typename real> static int list_steps(DeviceEnsemble *E, int nsteps) {
         if ((rc = enqueue_step<real>(E, true, nullptr)) != TFG_OK || (rc = finish(E)) != TFG_OK) return rc;
         const DeviceEnsemble::Status &now = *E->status;
         if (now.err[0] != 0 || now.err[1] != 0) break;
-        const int done = static_cast<int>(now.step - before.step), built = now.rebuilds - before.rebuilds;
+        const int done = static_cast<int>(now.step - before.step), served = now.served - before.served;
         if (done < 1 || done > left) return set_error(TFG_E_DEVICE, "list steps: the step counter is off");
         left -= done;
-        if (built > 0)
-            E->light_run = std::max(1, std::min(32, static_cast<int>(std::sqrt(8.0 * done / built))));
+        if (served > 0)
+            E->light_run = std::max(1, std::min(32, static_cast<int>(std::sqrt(8.0 * done / served))));
         else if (done > E->light_run)
             E->light_run = std::min(32, 2 * E->light_run);
     }

@@ -673,20 +673,17 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                             const int b0 = seg0 > 0 ? before : 0;
                             int pos = lbase + inc - c - b0;
                             const int *codes = s_slot + kb;
-                            // entry pos of particle si, then 64 ints further per entry
-                            int *lw = P.list + list_index(pos, si, P.lcap);
+                            int *lw = P.list + list_base(si, P.lcap);
                             while (m0) {
                                 const int t = __builtin_ctzll(m0);
                                 m0 &= m0 - 1ull;
-                                if (pos < P.lcap) *lw = codes[t];
-                                lw += 64;
+                                if (pos < P.lcap) lw[list_row(pos)] = codes[t];
                                 pos++;
                             }
                             while (m1) {
                                 const int t = __builtin_ctzll(m1);
                                 m1 &= m1 - 1ull;
-                                if (pos < P.lcap) *lw = codes[64 + t];
-                                lw += 64;
+                                if (pos < P.lcap) lw[list_row(pos)] = codes[64 + t];
                                 pos++;
                             }
                             lbase += last - b0;
@@ -939,7 +936,7 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                         const unsigned pad = static_cast<unsigned>(P.np) |
                                              (static_cast<unsigned>(kCentreCode) << kListSlotBits);
                         const int padded = min((lbase + kListBatch - 1) & ~(kListBatch - 1), P.lcap);
-                        for (int k = lbase; k < padded; k++) P.list[list_index(k, si, P.lcap)] = static_cast<int>(pad);
+                        for (int k = lbase; k < padded; k++) P.list[list_base(si, P.lcap) + list_row(k)] = static_cast<int>(pad);
                     }
                     continue;
                 }
@@ -1138,8 +1135,9 @@ __device__ inline double list_guard_r2(const KP<double> &, const SysDesc &, int,
 // the flux-only pass of the flux sub-steps (the role of
 // runner_dopair_fluxonly, tf_runner_dopair.cpp:334-412): pending flux only,
 // no forces, density or energies.  A workgroup covers up to kNbThreads
-// particles of one system and caches its pair descriptors, tables and the
-// the 125 build-cell shifts (in FP64) in LDS.  The pair test, the FP32 cutoff
+// particles of one system and holds the system's pair descriptors, tables
+// and the 125 build-cell shifts (in FP64) in LDS, copied from an image made
+// once (k_list_image).  The pair test, the FP32 cutoff
 // guard (band pairs decided in FP64 from the stored positions), the number
 // density and the table evaluation are those of the cell kernel.
 //
@@ -1155,7 +1153,8 @@ __device__ inline double list_guard_r2(const KP<double> &, const SysDesc &, int,
 // MULTI: the instance with several lanes per particle (small systems, and
 // table-only systems at any size); the other keeps one lane per particle
 // with no sub-lane bookkeeping.
-template <typename real, bool ENERGY, bool DPD = false, bool FLUX = false, bool FORCES = true, bool MULTI = false>
+typedef unsigned Entries __attribute__((ext_vector_type(kListBatch)));   // a batch of list entries
+template <typename real, bool ENERGY, bool DPD, bool FLUX, bool FORCES, bool MULTI>
 __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     using v4 = typename V<real>::v4;
     constexpr bool kGuarded = std::is_same<real, float>::value;
@@ -1169,34 +1168,25 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
         // for its rebuild; nothing writes these words during this kernel, and
         // the kernels after it take the decision from lflags[5].
         const bool go = P.err[0] == 0 && P.err[1] == 0 && P.lflags[4] == 0;
-        if (blockIdx.x == 0 && threadIdx.x == 0) P.lflags[5] = go ? 1 : 0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            P.lflags[5] = go ? 1 : 0;
+            P.lflags[7] = static_cast<int>(*P.step) + 1;
+        }
         if (!go) return;
     } else if (P.err[0] != 0) {
         return;   // halted (nothing writes the word during this kernel)
     }
     // Workgroups go to the 8 XCDs in turn: the workgroups of one XCD take
-    // consecutive particle blocks (the grid is a multiple of 8), so that the
-    // partner positions they gather meet in that XCD's L2.
+    // consecutive particle chunks (the grid is a multiple of 8), so that the
+    // partner positions they gather meet in that XCD's L2.  (Workgroups that
+    // take several chunks in turn were slower: the loop costs the FP32 pass 73
+    // spilled registers.)
     const int nblk = gridDim.x;
-    const int b = (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8;
-    const int4 lb = P.lblock[b];
+    const int4 lb = P.lblock[(blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8];
     const SysDesc &sd = P.sys[lb.x];
     const int nt = sd.ntypes;
-    v4 *s_pair = reinterpret_cast<v4 *>(s_dyn);
     // build-cell shifts by offset code: (x, y) at 16 code, (z, 0) kListShiftZ bytes further
-    double2 *s_sh = reinterpret_cast<double2 *>(s_dyn + P.nb.off_waves);
-    for (int t = threadIdx.x; t < sd.nslots; t += kNbThreads) write_pair_descriptor<real, true>(P, sd, t, P.nb.off_coef, s_pair);
-    cache_tables(P, sd, s_dyn + P.nb.off_coef, P.nb.coef_half);
-    for (int c = threadIdx.x; c < 125; c += kNbThreads) {
-        s_sh[c] = make_double2((c / 25 - 2) * sd.h[0], (c / 5 % 5 - 2) * sd.h[1]);
-        s_sh[kListShiftZ / 16 + c] = make_double2((c % 5 - 2) * sd.h[2], 0.0);
-    }
-    if (FLUX) {
-        for (int t = threadIdx.x; t < nt * nt; t += kNbThreads)
-            s_fmap[t] = make_int2(P.fluxmap[2 * (sd.flux_off + t)], P.fluxmap[2 * (sd.flux_off + t) + 1]);
-        for (int t = threadIdx.x; t < sd.nflux; t += kNbThreads) s_flux[t] = P.flux[sd.flux_first + t];
-    }
-    __syncthreads();
+    const double2 *s_sh = reinterpret_cast<const double2 *>(s_dyn + P.nb.off_waves);
 
     // P.lpp lanes per particle (a power of two; more than one in small
     // systems, to fill the device): sub-lane `sub` takes batches sub, sub +
@@ -1206,6 +1196,26 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     const int pl = MULTI ? static_cast<int>(threadIdx.x) >> P.lpp_log2 : static_cast<int>(threadIdx.x);
     const bool valid = pl < lb.z;
     const int i = lb.y + (valid ? pl : 0);
+    // The particles' own loads go before the wait for the system's data.
+    const v4 pi = P.xb[i];
+    const int2 mi = *reinterpret_cast<const int2 *>(&P.A.meta[i]);
+    // the near lists are read, else the lists as built
+    const bool near = P.sflags[3 * P.nsys + lb.x] != kListAll && P.sflags[4 * P.nsys + lb.x] == 0;
+    const int count = near ? P.ncount[i] : P.lcount[i];
+    const int n = valid ? (near ? count & 0xffff : min(count, P.lcap)) : 0;
+    // the sub-lane's first batch; batches are 64 particles' batches apart
+    const Entries *lp =
+        reinterpret_cast<const Entries *>(P.list + list_base(i, P.lcap)) + 64 * ((near ? count >> 16 : 0) + sub);
+    Entries en = __builtin_nontemporal_load(lp);
+    // the system's descriptors, tables and shifts as they lie in LDS
+    const uint4 *image = reinterpret_cast<const uint4 *>(P.limage + static_cast<size_t>(lb.x) * P.nb.total);
+    for (int t = threadIdx.x; t < P.nb.total / 16; t += kNbThreads) reinterpret_cast<uint4 *>(s_dyn)[t] = image[t];
+    if (FLUX) {
+        for (int t = threadIdx.x; t < nt * nt; t += kNbThreads)
+            s_fmap[t] = make_int2(P.fluxmap[2 * (sd.flux_off + t)], P.fluxmap[2 * (sd.flux_off + t) + 1]);
+        for (int t = threadIdx.x; t < sd.nflux; t += kNbThreads) s_flux[t] = P.flux[sd.flux_first + t];
+    }
+    __syncthreads();
     const real cut2 = kGuarded ? real(sd.cutoff2 * (1.0 + kGuard)) : real(sd.cutoff2);
     const real cut2_lo = kGuarded ? real(sd.cutoff2 * (1.0 - kGuard)) : real(sd.cutoff2);
     const bool binside = kGuarded && sd.binside != 0;
@@ -1214,12 +1224,9 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     const real w3 = real(0.75 * sd.w_self / (sd.cutoff2 * sd.cutoff));
     const real eps2 = eps_of<real>() * eps_of<real>();
 
-    const v4 pi = P.xb[i];
     const double pxd = static_cast<double>(pi.x), pyd = static_cast<double>(pi.y), pzd = static_cast<double>(pi.z);
-    const int2 mi = *reinterpret_cast<const int2 *>(&P.A.meta[i]);
     const int ti = mi.x & 0xffff;
     const int ti_row = ti * nt * kCol;
-    const int n = valid ? min(P.lcount[i], P.lcap) : 0;
     const int nbat = (n + kListBatch - 1) & ~(kListBatch - 1);   // the build padded the list to here
     real fx = 0, fy = 0, fz = 0, nd = 0, ep = 0, vir = 0;
     const int S = P.S;
@@ -1231,7 +1238,6 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     const long long tstep = sd.time0 + *P.step + P.step_ahead;
     const real dpd_delta = real(sd.inv_sqrt_dt);
     (void)tstep; (void)dpd_delta; (void)S;
-    const int *lp = P.list + list_index(kListBatch * sub, i, P.lcap);   // entry k at lp[64 (k - 4 sub)]
     // The entries of the next batch are loaded while this batch computes (they
     // stream from HBM); the partner positions of a batch are gathered at its
     // start.  The loads of the next batch are unconditional, so that the wait
@@ -1239,17 +1245,12 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     // they read lpp batches past it, inside the buffer (the allocation has
     // that slack), and are not used.  Entries are read once per step
     // (non-temporal: L2 stays with the gathers).
-    unsigned en[kListBatch];
-#pragma unroll
-    for (int u = 0; u < kListBatch; u++) en[u] = static_cast<unsigned>(__builtin_nontemporal_load(lp + 64 * u));
     const int nbat_mine = nbat - kListBatch * sub;   // the batches from this sub-lane's first
     for (int k0 = 0; k0 < nbat_mine; k0 += kListBatch * lpp) {
-        unsigned ev[kListBatch];
+        const Entries ev = en;
         v4 pv[kListBatch];
         v4 vv[DPD ? kListBatch : 1];
         int idv[kIds ? kListBatch : 1];
-#pragma unroll
-        for (int u = 0; u < kListBatch; u++) ev[u] = en[u];
 #pragma unroll
         for (int u = 0; u < kListBatch; u++) {
             const int j = static_cast<int>(ev[u] & kListSlotMask);
@@ -1261,9 +1262,8 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
         // memory counters retire in issue order: the gathers go first, so that
         // waiting for them never waits for the next batch's entries
         __builtin_amdgcn_sched_barrier(0);
-        lp += 64 * kListBatch * lpp;
-#pragma unroll
-        for (int u = 0; u < kListBatch; u++) en[u] = static_cast<unsigned>(__builtin_nontemporal_load(lp + 64 * u));
+        lp += 64 * lpp;
+        en = __builtin_nontemporal_load(lp);
 #pragma unroll
         for (int u = 0; u < kListBatch; u++) {
             const unsigned e = ev[u];
@@ -1406,7 +1406,7 @@ __device__ __forceinline__ void list_force_body(const KP<real> &P) {
     }
 }
 
-template <typename real, bool ENERGY, bool DPD = false, bool FLUX = false, bool FORCES = true, bool MULTI = false>
+template <typename real, bool ENERGY, bool DPD, bool FLUX, bool FORCES, bool MULTI>
 __global__ __launch_bounds__(kNbThreads) void k_list_force(KP<real> P) {
     list_force_body<real, ENERGY, DPD, FLUX, FORCES, MULTI>(P);
 }
@@ -1424,9 +1424,185 @@ template <typename real, bool DPD, bool FLUX> static const void *list_fn(bool en
     if (multi)
         return energy ? reinterpret_cast<const void *>(&k_list_force<real, true, DPD, FLUX, true, true>)
                       : reinterpret_cast<const void *>(&k_list_force<real, false, DPD, FLUX, true, true>);
-    return energy ? reinterpret_cast<const void *>(&k_list_force<real, true, DPD, FLUX>)
-                  : reinterpret_cast<const void *>(&k_list_force<real, false, DPD, FLUX>);
+    return energy ? reinterpret_cast<const void *>(&k_list_force<real, true, DPD, FLUX, true, false>)
+                  : reinterpret_cast<const void *>(&k_list_force<real, false, DPD, FLUX, true, false>);
 }
+
+// The near lists of the systems that make them in this step (k_tick_list):
+// the list entries within cutoff + near skin at the step's positions, in list
+// order, padded like the lists, in the lists' unused rows (a system without
+// room for them reads the lists).  The distance is the pair pass's.  A kernel
+// of its own, since a pair pass that also writes them needs 130 to 142 VGPRs
+// (three waves per SIMD) in every full step.  Blocks as in the pair pass.
+//
+// LANES: every sub-lane of a particle tests its batches, and a round's
+// entries are placed together, one 4-byte store each: for small systems,
+// where one lane per particle leaves the device idle.  Otherwise one lane per
+// particle, and the wave's entries go through a ring of kRing per lane in
+// LDS, from which it stores a batch of all its lanes as 1 KB in a row once
+// every lane has filled it.
+constexpr int kRing = 32;
+__device__ inline unsigned dummy_entry(int np) {
+    return static_cast<unsigned>(np) | (static_cast<unsigned>(kCentreCode) << kListSlotBits);
+}
+
+template <typename real, bool LANES> __global__ __launch_bounds__(kNbThreads) void k_near(KP<real> P) {
+    using v4 = typename V<real>::v4;
+    constexpr int kBatches = LANES ? 1 : 2;   // batches of a lane and round, loaded together
+    __shared__ double s_sh[3][125];
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    const int nblk = gridDim.x;
+    const int4 lb = P.lblock[(blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8];
+    if (P.sflags[3 * P.nsys + lb.x] != kListMakeNear || P.err[0] != 0) return;
+    const SysDesc &sd = P.sys[lb.x];
+    for (int c = threadIdx.x; c < 125; c += blockDim.x) {
+        s_sh[0][c] = (c / 25 - 2) * sd.h[0];
+        s_sh[1][c] = (c / 5 % 5 - 2) * sd.h[1];
+        s_sh[2][c] = (c % 5 - 2) * sd.h[2];
+    }
+    __syncthreads();
+    const int lpp = LANES ? P.lpp : 1, sub = static_cast<int>(threadIdx.x) & (lpp - 1);
+    const int pl = static_cast<int>(threadIdx.x) >> (LANES ? P.lpp_log2 : 0);
+    const bool valid = pl < lb.z;
+    const int i = lb.y + (valid ? pl : 0);
+    const v4 pi = P.xb[i];
+    const double px = static_cast<double>(pi.x), py = static_cast<double>(pi.y), pz = static_cast<double>(pi.z);
+    const real cutn2 = real(sd.cutn2);
+    const unsigned dummy = dummy_entry(P.np);
+    const int n = valid ? min(P.lcount[i], P.lcap) : 0;
+    const Entries *from = reinterpret_cast<const Entries *>(P.list + list_base(i, P.lcap));
+    // The wave's near lists start behind its longest list, at one row for all
+    // its lanes (rows of other waves' lanes are read with them).
+    int start = (n + kListBatch - 1) & ~(kListBatch - 1);
+    for (int o = 1; o < kWave; o <<= 1) start = max(start, __shfl_xor(start, o));
+    const int room = P.lcap - start;
+    int *to = P.list + list_base(i, P.lcap) + 64 * start;
+    const int last = (static_cast<int>(threadIdx.x) & (kWave - 1)) | (lpp - 1);   // the particle's last lane
+    int kept = 0;
+    // LANES: rounds while the particle's lanes have batches; else while any
+    // lane of the wave has
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    const Entries blank = {dummy, dummy, dummy, dummy};
+    // batch b of this lane's ring at ring[64 b], entry pos at batch pos / 4 % (kRing / 4)
+    Entries *ring = reinterpret_cast<Entries *>(s_dyn) + (threadIdx.x / kWave) * kWave * (kRing / kListBatch) + lane;
+    int flushed = 0;   // entries of each lane that have left the ring (a whole number of batches)
+    if (!LANES)
+        for (int b = 0; b < kRing / kListBatch; b++) ring[kWave * b] = blank;
+    auto flush = [&]() {   // the oldest batch: lanes that have nothing there store dummies
+        Entries &r = ring[kWave * (flushed / kListBatch % (kRing / kListBatch))];
+        if (valid && flushed < room) *reinterpret_cast<Entries *>(to + 64 * flushed) = r;
+        r = blank;
+        flushed += kListBatch;
+    };
+    for (int k0 = 0; LANES ? k0 < n : __any(k0 < n); k0 += kListBatch * kBatches * lpp) {
+        Entries ev[kBatches];
+        v4 pv[kBatches * kListBatch];
+#pragma unroll
+        for (int b = 0; b < kBatches; b++) {   // lists are padded to whole batches
+            const int k = k0 + kListBatch * (kBatches * sub + b);
+            ev[b] = Entries{dummy, dummy, dummy, dummy};
+            if (k < n) ev[b] = __builtin_nontemporal_load(from + 16 * k);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatches * kListBatch; u++) pv[u] = P.xb[ev[u / kListBatch][u % kListBatch] & kListSlotMask];
+        unsigned keep = 0;
+#pragma unroll
+        for (int u = 0; u < kBatches * kListBatch; u++) {
+            const unsigned e = ev[u / kListBatch][u % kListBatch];
+            const int c = static_cast<int>(e >> kListSlotBits);
+            const real dx = real(px - (static_cast<double>(pv[u].x) + s_sh[0][c]));
+            const real dy = real(py - (static_cast<double>(pv[u].y) + s_sh[1][c]));
+            const real dz = real(pz - (static_cast<double>(pv[u].z) + s_sh[2][c]));
+            const bool in = fma_of(dz, dz, fma_of(dy, dy, dx * dx)) <= cutn2;
+            if (LANES) {
+                keep |= (in ? 1u : 0u) << u;
+            } else if (in) {
+                if (kept >= flushed)
+                    reinterpret_cast<unsigned *>(&ring[kWave * (kept / kListBatch % (kRing / kListBatch))])[kept % kListBatch] = e;
+                else if (kept < room)   // its batch had to leave before this lane filled it
+                    to[list_row(kept)] = static_cast<int>(e);
+                kept++;
+            }
+        }
+        if (!LANES) {
+            // batches that every lane has filled or has no more entries for,
+            // and the oldest when a lane might run out of ring
+            while (__all(kept >= flushed + kListBatch || k0 + kListBatch * kBatches >= n) && __any(kept > flushed)) flush();
+            while (__any(kept - flushed > kRing - kListBatch * kBatches)) flush();
+            continue;
+        }
+        if (LANES) {
+            const int c = __popc(keep);
+            int inc = c;
+            for (int o = 1; o < lpp; o <<= 1) {
+                const int y = __shfl_up(inc, o);
+                if (sub >= o) inc += y;
+            }
+            int at = kept + inc - c;
+#pragma unroll
+            for (int u = 0; u < kListBatch; u++)
+                if (keep & (1u << u)) {
+                    if (at < room) to[list_row(at)] = static_cast<int>(ev[0][u]);
+                    at++;
+                }
+            kept += __shfl(inc, last);
+        }
+    }
+    if (!valid || sub != 0) return;
+    if (kept > room) {   // no room behind the lists: outlived at once
+        P.sflags[4 * P.nsys + lb.x] = 1;
+        P.lflags[4] = 1;
+        return;
+    }
+    P.ncount[i] = kept | (start / kListBatch) << 16;
+    if (LANES)   // (a room of whole batches holds the padding)
+        for (int k = kept; k & (kListBatch - 1); k++) to[list_row(k)] = static_cast<int>(dummy);
+}
+
+template <typename real> int run_near(DeviceEnsemble *E, const KP<real> &P) {
+    if (E->lpp > 2)
+        hipLaunchKernelGGL((k_near<real, true>), dim3(E->nlblocks), dim3(kNbThreads), 0, E->stream, P);
+    else
+        hipLaunchKernelGGL((k_near<real, false>), dim3(E->nlblocks), dim3(kNbThreads / E->lpp),
+                           kNbThreads / E->lpp * kRing * static_cast<int>(sizeof(int)), E->stream, P);
+    return launch_error("near lists");
+}
+
+template int run_near<float>(DeviceEnsemble *, const KP<float> &);
+template int run_near<double>(DeviceEnsemble *, const KP<double> &);
+
+// The LDS contents of the pair pass for each system.  Building them in the
+// pass took a chain of four dependent loads (system, slot, potential,
+// coefficients) at the start of every workgroup.
+template <typename real> __global__ __launch_bounds__(kNbThreads) void k_list_image(KP<real> P, unsigned char *image) {
+    using v4 = typename V<real>::v4;
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    const SysDesc &sd = P.sys[blockIdx.x];
+    uint4 *s_all = reinterpret_cast<uint4 *>(s_dyn);
+    for (int t = threadIdx.x; t < P.nb.total / 16; t += kNbThreads) s_all[t] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    for (int t = threadIdx.x; t < sd.nslots; t += kNbThreads)
+        write_pair_descriptor<real, true>(P, sd, t, P.nb.off_coef, reinterpret_cast<v4 *>(s_dyn));
+    cache_tables(P, sd, s_dyn + P.nb.off_coef, P.nb.coef_half);
+    double2 *s_sh = reinterpret_cast<double2 *>(s_dyn + P.nb.off_waves);
+    for (int c = threadIdx.x; c < 125; c += kNbThreads) {
+        s_sh[c] = make_double2((c / 25 - 2) * sd.h[0], (c / 5 % 5 - 2) * sd.h[1]);
+        s_sh[kListShiftZ / 16 + c] = make_double2((c % 5 - 2) * sd.h[2], 0.0);
+    }
+    __syncthreads();
+    uint4 *out = reinterpret_cast<uint4 *>(image + static_cast<size_t>(blockIdx.x) * P.nb.total);
+    for (int t = threadIdx.x; t < P.nb.total / 16; t += kNbThreads) out[t] = s_all[t];
+}
+
+template <typename real> int run_list_image(DeviceEnsemble *E, const KP<real> &P) {
+    KP<real> Q = P;
+    Q.nb = E->nbl;
+    hipLaunchKernelGGL(k_list_image<real>, dim3(E->nsys), dim3(kNbThreads), E->nbl.total, E->stream, Q, E->d_limage);
+    return launch_error("list image");
+}
+
+template int run_list_image<float>(DeviceEnsemble *, const KP<float> &);
+template int run_list_image<double>(DeviceEnsemble *, const KP<double> &);
 
 template <typename real> int run_list_force(DeviceEnsemble *E, const KP<real> &P) {
     KP<real> Q = P;
@@ -1445,7 +1621,7 @@ template <typename real> int run_list_flux(DeviceEnsemble *E, const KP<real> &P)
     Q.nb = E->nbl;
     void *args[] = {&Q};
     const void *fn = E->lpp > 1 ? reinterpret_cast<const void *>(&k_list_force<real, false, false, true, false, true>)
-                                : reinterpret_cast<const void *>(&k_list_force<real, false, false, true, false>);
+                                : reinterpret_cast<const void *>(&k_list_force<real, false, false, true, false, false>);
     const hipError_t e = hipLaunchKernel(fn, dim3(E->nlblocks), dim3(kNbThreads), args, E->nbl.total, E->stream);
     if (e != hipSuccess) return set_error(TFG_E_DEVICE, std::string("list flux: ") + hipGetErrorString(e));
     return launch_error("list flux");
