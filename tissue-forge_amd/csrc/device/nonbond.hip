@@ -104,6 +104,16 @@ __device__ inline double dist2(double4 a, double4 b) {
     return __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
 }
 
+// Whether distance r is in the guard's band around a range end b.  The
+// subtraction is not contracted with the product that made r, for the same
+// reason: fused in the loop and not in the rescan it dropped pairs at the
+// band's edge.
+template <typename real> __device__ inline bool near_end(real r, real b) {
+#pragma clang fp contract(off)
+    const real d = r - b;
+    return fabs(d) <= real(2.0 * kGuard) * b;
+}
+
 __device__ inline float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ inline double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
 // the 32-bit word holding a value's sign bit (bit 31)
@@ -466,7 +476,7 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                         real tdx = dx, tdy = dy, tdz = dz, tr2 = r2, tir = ir, traw = r_raw;
                         image(qt, mt, tdx, tdy, tdz, tr2, tir, traw, k);
                         const real rt = transformed(traw, mt, a2.x, k);
-                        band = band || ((mt & kMetaBInside) && fabs(rt - a0.y) <= real(2.0 * kGuard) * a0.y);
+                        band = band || ((mt & kMetaBInside) && near_end(rt, a0.y));
                         const int next = EXT ? real_bits_as_int(a2.w) : 0;
                         if (next == 0) break;
                         qt = reinterpret_cast<const v4 *>(s_dyn + next * kCol);
