@@ -24,7 +24,17 @@ constexpr int kWave = 64;
 constexpr int kMaxTypes = 8;          // type pairs cached in LDS by the pair kernel
 constexpr int kMaxSpecies = 8;        // TF_SIMD_SIZE
 constexpr int kMaxFluxEntries = 64;   // flux entries per system
-constexpr int kMaxSpanZ = 3;          // cells of cutoff along z per direction
+// Cell pass of crowded systems (more than kShareMean particles per cell on
+// average at the upload): a cell of more than kShareAbove particles is one
+// workgroup's.  One wave per cell leaves such systems with few waves, each
+// long: 8,000 particles in 216 cells 203 us a step, shared 97; 200,000 in
+// 6,859 cells 365 -> 340.  At 16 per cell sharing leaves a lane too few
+// candidates (1,000,000 particles 0.80 -> 1.53 ms), so those keep the wave.
+// The rule looks at the system alone, so that its results do not depend on
+// the ensemble it is in.
+constexpr double kShareMean = 20.0;
+constexpr int kShareAbove = 12;
+constexpr int kMaxSpan = 3;           // cells of cutoff per direction
 // FP32 path: pairs within this relative band of the cutoff (or of a table end
 // below it) are decided in FP64 by the pair kernel.
 constexpr double kGuard = 2e-6;
@@ -33,8 +43,8 @@ constexpr double kGuard = 2e-6;
 struct SysDesc {
     int cdim[3];
     int ncells, cell_off, p_off, np, ntypes;
-    int nstencil, stencil_off;   // columns (ox, oy) of the neighbour stencil
-    int span_z;                  // z extent of every column: -span_z .. span_z
+    int share_above;   // cell pass: a cell of more particles is one workgroup's, not one wave's
+    int nstencil, stencil_off;   // cells of the neighbour stencil (cell codes)
     int pot_off, nslots;          // descriptor slots (int2: potential, next slot) from pot_off
     int type_off;
     int sum_all;                  // a sum evaluates every constituent (else up to the first in range)
@@ -61,7 +71,7 @@ struct SysDesc {
     // Neighbour lists: the build stencil (cells within cutoff + skin, as
     // list codes) covers cutoff + skin; a particle displaced by more than
     // skin / 2 since the build requests a rebuild.
-    int nstencil_b, stencil_off_b, span_z_b;
+    int nstencil_b, stencil_off_b;
     double cutb2;        // (cutoff + skin)^2, widened by a relative 1e-5
     double skin_half2;   // (skin / 2)^2, narrowed by a relative 1e-4
     // Near lists: the list entries within cutoff + near skin, kept until a
@@ -93,6 +103,12 @@ constexpr int kNearLife = 4, kNearRetry = 16, kNearRetryMost = 256;
 constexpr int kNearMostCap = 65535;   // entries per particle (ncount's fields)
 constexpr int kNearShare = 8;   // age from which near lists are renewed with another system's
 constexpr float kListFar = 1.0e6f;
+// Neighbour cell of the cell pass, offsets within kMaxSpan: ox, oy, oz ascending.
+constexpr int kCodeSide = 2 * kMaxSpan + 1;
+__host__ __device__ inline int cell_code(int ox, int oy, int oz) {
+    return ((ox + kMaxSpan) * kCodeSide + (oy + kMaxSpan)) * kCodeSide + (oz + kMaxSpan);
+}
+constexpr int kOwnCell = (kMaxSpan * kCodeSide + kMaxSpan) * kCodeSide + kMaxSpan;   // cell_code(0, 0, 0)
 constexpr int kMaxBuildCells = 128;    // build stencil cells (at most 5^3)
 // Entry k of particle i: tiles of 64 particles of lcap * 256 bytes, inside a
 // tile batch by batch and a batch's particles in turn, so that a lane reads
@@ -163,13 +179,14 @@ struct NbLayout {
     int waves, chunk;
     int off_coef, coef_half, off_waves, region;
     int off_id, off_slot, off_vel, off_rad, off_sp;
+    int off_seg, off_mark;   // cell pass: segment table of the stencil, marks of segment starts
     int total;
 };
 
 template <typename real> struct KP {
     const SysDesc *sys;
     const int *cell_sys;
-    const int *stencil;   // 2 ints (ox, oy) per stencil column
+    const int *stencil;   // cell codes of the pair pass, list codes of the list build
     const PotDesc<real> *pots;
     const int2 *slots;    // per system: descriptor slot -> (potential, next slot or 0)
     const real *coef;
@@ -202,6 +219,7 @@ template <typename real> struct KP {
     int step_ahead;   // 1 when forces are evaluated outside a step (time + 1)
     int coef_lds;     // 1 when every system's pair tables fit the LDS cache
     NbLayout nb;
+    NbLayout nbs;     // cell pass: the staging area as one region, shared by a workgroup's waves
     // Neighbour lists (null and 0 without them).
     int list_mode;                    // (updates write buffer A in place)
     int light;                        // a light step: no binning, no build, skipped while a rebuild is due

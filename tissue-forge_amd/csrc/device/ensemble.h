@@ -71,6 +71,7 @@ struct DeviceEnsemble {
     int nr_fluxsteps = 1;                   // shared as well
     int coef_lds_bytes = 0;   // table bytes cached in LDS by the pair kernel (0: read from global)
     NbLayout nb{};            // LDS layout of the pair kernel
+    NbLayout nbs{};           // its staging area as one region, for cells that a workgroup shares
     NbLayout nbb{};           // LDS layout of the list-build variant
     NbLayout nbl{};           // LDS of the list pair kernel (off_coef: tables, off_waves: cell offsets)
     bool list_mode = false;   // neighbour lists in use (every member asked for them and can use them)
@@ -84,6 +85,7 @@ struct DeviceEnsemble {
     int *d_list = nullptr, *d_lcount = nullptr, *d_cid0 = nullptr, *d_lflags = nullptr, *d_sflags = nullptr;
     int *d_ncount = nullptr;
     void *xb = nullptr, *x0 = nullptr, *xn = nullptr;
+    int nb_cells = 4;         // cells of a pair-kernel workgroup
     int nonbond_resident = 0; // pair-kernel workgroups resident on the device at once
     LaunchShape shape;
     Buffers buf;
@@ -167,11 +169,12 @@ struct DeviceEnsemble {
         const int cap = shape.stream_blocks > 0 ? shape.stream_blocks : cus * 8;
         return want < 1 ? 1 : (want < cap ? want : cap);
     }
-    // Default: one cell per wave (the hardware dispatcher balances the uneven
+    // Default: one cell per wave, or per workgroup of crowded cells (the hardware dispatcher balances the uneven
     // cells; measured faster than persistent ranges on 2M- and 2.6M-particle
     // systems).
-    int nonbond_grid() const {
-        const int want = (ncells + nb.waves - 1) / (nb.waves > 0 ? nb.waves : 1);
+    int nonbond_grid() const { return grid_of((ncells + nb_cells - 1) / nb_cells); }
+    int build_grid() const { return grid_of((ncells + nb.waves - 1) / (nb.waves > 0 ? nb.waves : 1)); }   // one cell per wave
+    int grid_of(int want) const {
         const int g = shape.nonbond_blocks > 0 && shape.nonbond_blocks < want ? shape.nonbond_blocks : want;
         return g < 1 ? 1 : g;
     }
@@ -202,7 +205,7 @@ template <typename real> int run_sync(DeviceEnsemble *E, const KP<real> &P, bool
 int run_count(DeviceEnsemble *E);
 template <typename real> int run_nonbond(DeviceEnsemble *E, const KP<real> &P);
 // Chooses the LDS layout and the resident grid of the pair kernel.
-template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_types, int max_coef);
+template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_types, int max_coef, int max_stencil);
 // update: 0 forces only, 1 forward-Euler update, 2..5 Runge-Kutta stage 1..4.
 template <typename real> int run_advance(DeviceEnsemble *E, const KP<real> &P, int update);
 // Neighbour lists: the build (a variant of the pair kernel over the wider

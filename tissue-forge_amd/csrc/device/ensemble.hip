@@ -3,6 +3,7 @@
 #include "ensemble.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -88,6 +89,7 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy) {
     P.step_ahead = 0;
     P.coef_lds = E->coef_lds_bytes > 0 ? 1 : 0;
     P.nb = E->nb;
+    P.nbs = E->nbs;
     P.list_mode = E->list_mode ? 1 : 0;
     P.light = 0;
     P.lpp = E->lpp;
@@ -377,7 +379,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     std::vector<std::vector<int>> remaps(nsys);
     bool list_ok = E->integrator == INTEG_FORWARD_EULER;   // neighbour lists for every member
     int lcap = 0;
-    int np = 0, nc = 0, max_coef = 0;
+    int np = 0, nc = 0, max_coef = 0, max_stencil = 0;
     for (int s = 0; s < nsys; s++) {
         Engine &e = *E->engines[s];
         SysDesc &d = sys[s];
@@ -396,24 +398,19 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         d.p_off = np;
         d.np = static_cast<int>(e.parts.size());
         d.ntypes = nt;
-        // Neighbour stencil as columns (ox, oy) spanning z in [-span_z, span_z]:
-        // a column is kept when its closest cell is inside the cutoff (the
-        // task cull of tfSpace.cpp:949-954 restricted to x and y); cells of a
-        // kept column that the full cull would drop are beyond the cutoff and
-        // only cost distance tests.
-        if (e.geom.span[2] > kMaxSpanZ)
-            return set_error(TFG_E_RANGE, "the cutoff spans more than 3 cells along z");
-        d.span_z = e.geom.span[2];
-        d.stencil_off = static_cast<int>(stencil.size() / 2);
-        for (int ox = -e.geom.span[0]; ox <= e.geom.span[0]; ox++)
-            for (int oy = -e.geom.span[1]; oy <= e.geom.span[1]; oy++) {
-                const double lx = e.geom.h[0] * std::fmax(std::abs(ox) - 1, 0);
-                const double ly = e.geom.h[1] * std::fmax(std::abs(oy) - 1, 0);
-                if (lx * lx + ly * ly > e.geom.cutoff2) continue;
-                stencil.push_back(ox);
-                stencil.push_back(oy);
-            }
-        d.nstencil = static_cast<int>(stencil.size() / 2) - d.stencil_off;
+        // Crowded systems (more than kShareMean particles per cell): the whole
+        // workgroup takes each cell of more than kShareAbove.
+        d.share_above = d.np > kShareMean * d.ncells ? kShareAbove : INT_MAX;
+        // Neighbour stencil: the cells whose closest point is inside the cutoff
+        // (the task cull of tfSpace.cpp:949-954), as cell codes.
+        for (int k = 0; k < 3; k++)
+            if (e.geom.span[k] > kMaxSpan)
+                return set_error(TFG_E_RANGE, std::string("the cutoff spans more than 3 cells along ") + "xyz"[k]);
+        d.stencil_off = static_cast<int>(stencil.size());
+        for (size_t k = 0; k < e.geom.stencil.size(); k += 3)
+            stencil.push_back(cell_code(e.geom.stencil[k], e.geom.stencil[k + 1], e.geom.stencil[k + 2]));
+        d.nstencil = static_cast<int>(stencil.size()) - d.stencil_off;
+        max_stencil = std::max(max_stencil, d.nstencil);
         // Neighbour lists: build stencil for cutoff + skin (at most two cells
         // per axis), the build radius widened and the rebuild threshold
         // narrowed by small margins.  Along a periodic axis the box must be
@@ -431,8 +428,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
                 if (sb[k] > 2 || ((per >> k & 1u) && e.geom.cdim[k] * e.geom.h[k] <= 2.0 * rcs * (1.0 + 1e-6)))
                     list_ok = false;
             }
-            d.span_z_b = sb[2];
-            d.stencil_off_b = static_cast<int>(stencil.size() / 2);
+            d.stencil_off_b = static_cast<int>(stencil.size());
             // The cells whose closest point is within cutoff + skin (the full
             // cell cull), as list codes, one per stencil entry.
             for (int ox = -sb[0]; ox <= sb[0]; ox++)
@@ -443,9 +439,8 @@ template <typename real> static int upload(DeviceEnsemble *E) {
                         const double lz = e.geom.h[2] * std::fmax(std::abs(oz) - 1, 0);
                         if (lx * lx + ly * ly + lz * lz > rcs * rcs) continue;
                         stencil.push_back(list_code(ox, oy, oz));
-                        stencil.push_back(0);
                     }
-            d.nstencil_b = static_cast<int>(stencil.size() / 2) - d.stencil_off_b;
+            d.nstencil_b = static_cast<int>(stencil.size()) - d.stencil_off_b;
             d.cutb2 = rcs * rcs * (1.0 + 1e-5);
             const double half = 0.5 * e.verlet_skin * (1.0 - 1e-4);
             d.skin_half2 = half * half;
@@ -604,6 +599,10 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     E->np = np;
     E->ncells = nc;
     E->sys = sys;
+    long long shared_cells = 0;
+    for (const SysDesc &d : sys)
+        if (d.share_above < INT_MAX) shared_cells += d.ncells;
+    E->nb_cells = 2 * shared_cells > nc ? 1 : 4;
     int max_np = 1;
     for (const SysDesc &d : sys) max_np = std::max(max_np, d.np);
     E->max_sys_blocks = (max_np + energy_tile() - 1) / energy_tile();
@@ -614,7 +613,7 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     E->list_mode = list_ok && !E->no_alloc && !E->has_ext && np + 1 < (1 << kListSlotBits) &&
                    static_cast<size_t>(max_coef) * sizeof(real) <= 16384;
     E->lcap = E->list_mode ? lcap : 0;
-    int rc = nonbond_setup<real>(E, max_nt, max_coef);
+    int rc = nonbond_setup<real>(E, max_nt, max_coef, max_stencil);
     if (rc != TFG_OK) return rc;
     if (E->list_mode && max_coef > 0 && E->coef_lds_bytes == 0) E->list_mode = false;
     // List pass blocks of 256 / lpp particles; lpp lanes per particle while
@@ -1199,7 +1198,8 @@ int ensemble_autotune(DeviceEnsemble *E, int reps, int *blocks_out, int *stream_
         return best;
     };
     const int res = std::max(1, E->nonbond_resident);
-    const int most = std::max(1, (E->ncells + E->nb.waves - 1) / E->nb.waves);
+    const int most =
+        std::max(1, E->list_mode ? (E->ncells + E->nb.waves - 1) / E->nb.waves : (E->ncells + E->nb_cells - 1) / E->nb_cells);
     std::vector<int> cand;
     for (int c : {res / 2, res, 2 * res, 3 * res, 4 * res, most})
         if (c >= 1 && c <= most && std::find(cand.begin(), cand.end(), c) == cand.end()) cand.push_back(c);

@@ -7,8 +7,9 @@
 // tf_flux_eval.h:48-103), and of the CUDA sort/self/pair kernels
 // (tfRunner_cuda.cu:2469-2845).
 //
-// Work unit: one wave per cell of i particles.  A workgroup of kNbWaves waves
-// owns a contiguous range of cells (workgroups of one XCD own neighbouring
+// Work unit: one wave per cell of i particles (crowded systems: one workgroup
+// per cell, whose waves stage together and take a part of its particles
+// each).  A workgroup of kNbWaves waves owns a contiguous range of cells (workgroups of one XCD own neighbouring
 // ranges, so their stencils meet in that XCD's L2); its waves take the cells
 // of the range in turn and share the pair descriptors and table
 // coefficients of the current system in LDS.  Each wave stages the particles
@@ -142,7 +143,7 @@ static inline int align16(int b) { return (b + 15) & ~15; }
 // staging region per wave (positions, ids, velocities, radii, species).
 template <typename real>
 NbLayout nb_layout(int max_nt, int coef_lds_count, int S, bool dpd, bool flux, bool radius, int max_chunk,
-                   bool build = false) {
+                   bool build = false, int max_stencil = 0, NbLayout *shared = nullptr) {
     using v4 = typename V<real>::v4;
     // ids: DPD noise and flux roles need the partner's id, periodic images
     // orient the pair by the lower id
@@ -169,6 +170,10 @@ NbLayout nb_layout(int max_nt, int coef_lds_count, int S, bool dpd, bool flux, b
         if (radius) b += align16(chunk * static_cast<int>(sizeof(real)));
         o->off_sp = b;
         if (flux) b += align16(chunk * S * static_cast<int>(sizeof(real)));
+        o->off_seg = b;
+        b += align16(3 * max_stencil * 4);
+        o->off_mark = b;
+        b += align16(chunk / 32 * 4);
         // the slice reduction reuses the region: 64 lanes x (6 + S) values
         return std::max(b, kWave * (6 + S) * static_cast<int>(sizeof(real)));
     };
@@ -177,6 +182,12 @@ NbLayout nb_layout(int max_nt, int coef_lds_count, int S, bool dpd, bool flux, b
     L.chunk = chunk;
     L.region = region(chunk, &L);
     L.total = L.off_waves + kNbWaves * L.region;
+    if (shared) {   // the waves' regions as one, of as many entries as they hold
+        *shared = L;
+        int most = kNbWaves * chunk;
+        while (region(most, shared) > kNbWaves * L.region) most -= kWave;
+        shared->chunk = most;
+    }
     return L;
 }
 
@@ -274,23 +285,9 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform in the wave
     const int lane = threadIdx.x & (kWave - 1);
     const int S = P.S;
-    const int chunk = P.nb.chunk;
     v4 *s_pair = reinterpret_cast<v4 *>(s_dyn);
-    unsigned char *region = s_dyn + P.nb.off_waves + wid * P.nb.region;
-    v4 *s_pos = reinterpret_cast<v4 *>(region);
-    int *s_id = reinterpret_cast<int *>(region + P.nb.off_id);
-    // BUILD (no ids there): the staged index of each i particle itself, then
-    // the segment table of the build stencil (ends, slot bases, offset codes)
-    int *s_self = reinterpret_cast<int *>(region + P.nb.off_id);
-    int *s_bend = s_self + kWave;
-    int *s_bbase = s_bend + kMaxBuildCells;
-    int *s_bcode = s_bbase + kMaxBuildCells;
-    (void)s_self; (void)s_bend; (void)s_bbase; (void)s_bcode;
-    int *s_slot = reinterpret_cast<int *>(region + P.nb.off_slot);
-    v4 *s_vel = reinterpret_cast<v4 *>(region + P.nb.off_vel);
-    real *s_rad = reinterpret_cast<real *>(region + P.nb.off_rad);
-    real *s_sp = reinterpret_cast<real *>(region + P.nb.off_sp);
-    real *s_red = reinterpret_cast<real *>(region);
+    unsigned char *wave_region = s_dyn + P.nb.off_waves + wid * P.nb.region;
+    real *s_red = reinterpret_cast<real *>(wave_region);
 
     // Workgroups are dispatched to the XCDs in turn; give the workgroups of
     // one XCD consecutive cell ranges.
@@ -354,10 +351,43 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
         const real dpd_delta = real(sd.inv_sqrt_dt);
         const real eps2 = eps_of<real>() * eps_of<real>();
 
-        for (int c = seg + wid; c < seg_end; c += kNbWaves) {
+        // The shared cells first, by all waves together, then each wave its
+        // own of the others (the list build: only those).
+        for (int phase = BUILD ? 1 : 0; phase < 2; phase++)
+        for (int c = phase ? seg + wid : seg; c < seg_end; c += phase ? kNbWaves : 1) {
             const int i0 = P.start[c];
             const int ni = P.start[c + 1] - i0;
-            if (ni == 0) continue;
+            const bool share = !BUILD && phase == 0;
+            if (ni == 0 || (!BUILD && (ni > sd.share_above) != share)) continue;
+            // the staging region: the wave's own, or the workgroup's
+            const NbLayout &lay = share ? P.nbs : P.nb;
+            const int chunk = lay.chunk;
+            unsigned char *region = share ? s_dyn + P.nb.off_waves : wave_region;
+            v4 *s_pos = reinterpret_cast<v4 *>(region);
+            int *s_id = reinterpret_cast<int *>(region + lay.off_id);
+            // BUILD (no ids there): the staged index of each i particle itself, then
+            // the segment table of the build stencil (ends, slot bases, offset codes)
+            int *s_self = reinterpret_cast<int *>(region + lay.off_id);
+            int *s_bend = s_self + kWave;
+            int *s_bbase = s_bend + kMaxBuildCells;
+            int *s_bcode = s_bbase + kMaxBuildCells;
+            (void)s_self; (void)s_bend; (void)s_bbase; (void)s_bcode; (void)s_id;
+            int *s_slot = reinterpret_cast<int *>(region + lay.off_slot);
+            v4 *s_vel = reinterpret_cast<v4 *>(region + lay.off_vel);
+            real *s_rad = reinterpret_cast<real *>(region + lay.off_rad);
+            real *s_sp = reinterpret_cast<real *>(region + lay.off_sp);
+            (void)s_vel; (void)s_rad; (void)s_sp;
+            const int tfirst = share ? static_cast<int>(threadIdx.x) : lane;   // staging threads
+            const int tstep_of = share ? kNbThreads : kWave;
+            auto sync = [&]() {
+                if (share)
+                    __syncthreads();
+                else
+                    wave_sync();
+            };
+            // particles of a wave and pass, and of a pass
+            const int group = share ? min(kWave, (ni + kNbWaves - 1) / kNbWaves) : kWave;
+            const int per_pass = share ? group * kNbWaves : kWave;
             int loc[3];
             cell_loc(c - sd.cell_off, sd, loc);
             // BUILD: the segment table of this cell's build stencil.  One lane
@@ -365,6 +395,65 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
             // together); an inclusive scan gives each cell's end in the flat
             // candidate order, so candidate t of the flat order is slot
             // s_bbase[sg] + t of the cell sg with s_bend[sg - 1] <= t < s_bend[sg].
+            // The first slot and the count of the stencil cell at offset o
+            // (none beyond a non-periodic face: space_init's task list skips
+            // it, tfSpace.cpp:913-944).
+            auto stencil_cell = [&](const int (&o)[3], int *first, int *cnt) {
+                int nb[3];
+                bool inside = true;
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    nb[k] = loc[k] + o[k];
+                    if (sd.periodic & (1 << k)) {
+                        nb[k] += nb[k] < 0 ? sd.cdim[k] : 0;
+                        nb[k] -= nb[k] >= sd.cdim[k] ? sd.cdim[k] : 0;
+                    } else if (nb[k] < 0 || nb[k] >= sd.cdim[k]) {
+                        inside = false;
+                    }
+                }
+                if (inside) {
+                    const int cc = sd.cell_off + (nb[0] * sd.cdim[1] + nb[1]) * sd.cdim[2] + nb[2];
+                    *first = P.start[cc];
+                    *cnt = P.start[cc + 1] - *first;
+                }
+            };
+            // The cell pass: the non-empty stencil cells in order, each with
+            // its first candidate (the candidates of all cells in a row), the
+            // slot less candidate, and its code.  One lane per cell, so that
+            // the loads of all cells are in flight together.
+            int *s_seg = reinterpret_cast<int *>(region + lay.off_seg);
+            unsigned *s_mark = reinterpret_cast<unsigned *>(region + lay.off_mark);
+            int nseg = 0, total = 0, self_base = 0;   // self_base: candidate less slot in the own cell
+            (void)s_seg; (void)s_mark; (void)self_base;
+            if constexpr (!BUILD) {
+                for (int h0 = 0; h0 < sd.nstencil; h0 += kWave) {
+                    int cnt = 0, first = 0, code = -1;
+                    if (h0 + lane < sd.nstencil) {
+                        code = P.stencil[sd.stencil_off + h0 + lane];
+                        const int o[3] = {code / (kCodeSide * kCodeSide) - kMaxSpan, code / kCodeSide % kCodeSide - kMaxSpan,
+                                          code % kCodeSide - kMaxSpan};
+                        stencil_cell(o, &first, &cnt);
+                    }
+                    int inc = cnt;
+#pragma unroll
+                    for (int o = 1; o < kWave; o <<= 1) {
+                        const int y = __shfl_up(inc, o);
+                        if (lane >= o) inc += y;
+                    }
+                    const int off = total + inc - cnt;
+                    const unsigned long long some = __ballot(cnt > 0), own = __ballot(code == kOwnCell);
+                    if (cnt > 0) {
+                        int *e = s_seg + 3 * (nseg + __popcll(some & ((1ull << lane) - 1ull)));
+                        e[0] = off;
+                        e[1] = first - off;
+                        e[2] = code;
+                    }
+                    if (own != 0ull) self_base = __shfl(off - first, __builtin_ctzll(own));
+                    nseg += __popcll(some);
+                    total += __shfl(inc, kWave - 1);
+                }
+                sync();
+            }
             int btotal = 0;
             if constexpr (BUILD) {
                 int carry = 0;
@@ -373,26 +462,9 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                     const int sgi = half * kWave + lane;
                     int cnt = 0, first = 0, code = kCentreCode;
                     if (sgi < sd.nstencil_b) {
-                        code = P.stencil[2 * (sd.stencil_off_b + sgi)];
+                        code = P.stencil[sd.stencil_off_b + sgi];
                         const int o[3] = {code / 25 - 2, code / 5 % 5 - 2, code % 5 - 2};
-                        int nb[3];
-                        bool inside = true;
-#pragma unroll
-                        for (int k = 0; k < 3; k++) {
-                            nb[k] = loc[k] + o[k];
-                            // beyond a non-periodic face there is no neighbour
-                            if (sd.periodic & (1 << k)) {
-                                nb[k] += nb[k] < 0 ? sd.cdim[k] : 0;
-                                nb[k] -= nb[k] >= sd.cdim[k] ? sd.cdim[k] : 0;
-                            } else if (nb[k] < 0 || nb[k] >= sd.cdim[k]) {
-                                inside = false;
-                            }
-                        }
-                        if (inside) {
-                            const int cc = sd.cell_off + (nb[0] * sd.cdim[1] + nb[1]) * sd.cdim[2] + nb[2];
-                            first = P.start[cc];
-                            cnt = P.start[cc + 1] - first;
-                        }
+                        stencil_cell(o, &first, &cnt);
                     }
                     int inc = cnt;
 #pragma unroll
@@ -410,12 +482,15 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                 wave_sync();
             }
 
-            for (int ib = 0; ib < ni; ib += kWave) {
-                const int nib = min(kWave, ni - ib);
+            for (int pass = 0; pass < ni; pass += per_pass) {
+                const int ib = pass + (share ? min(wid * group, ni - 1 - pass) : 0);
+                // (a wave past the last particle only stages)
+                const bool idle = share && pass + wid * group >= ni;
+                const int nib = idle ? 1 : min(group, ni - ib);
                 const int slices = kWave / nib;
                 const int il = lane / slices;
                 const int sl = lane - il * slices;
-                const bool active = il < nib;
+                const bool active = il < nib && !idle;
                 const int ii = ib + (active ? il : 0);   // index of the i particle in its cell
                 const int si = i0 + ii;
                 const v4 pi4 = P.A.pos[si];
@@ -847,94 +922,93 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                         }
                     }
                 } else {
-                    const int sz = sd.span_z;
-                    const int nst = sd.nstencil;
-                    const int st_off = sd.stencil_off;
-                    for (int col = 0; col < nst; col++) {
-                        const int ox = P.stencil[2 * (st_off + col)];
-                        const int oy = P.stencil[2 * (st_off + col) + 1];
-                        const int szc = sz;
-                        int n0 = loc[0] + ox;
-                        int n1 = loc[1] + oy;
-                        // beyond a non-periodic face there is no neighbour
-                        // (space_init's task list skips it, tfSpace.cpp:913-944)
-                        if (!(sd.periodic & 1) && (n0 < 0 || n0 >= sd.cdim[0])) continue;
-                        if (!(sd.periodic & 2) && (n1 < 0 || n1 >= sd.cdim[1])) continue;
-                        n0 += n0 < 0 ? sd.cdim[0] : 0;
-                        n0 -= n0 >= sd.cdim[0] ? sd.cdim[0] : 0;
-                        n1 += n1 < 0 ? sd.cdim[1] : 0;
-                        n1 -= n1 >= sd.cdim[1] ? sd.cdim[1] : 0;
-                        const int colbase = sd.cell_off + (n0 * sd.cdim[1] + n1) * sd.cdim[2];
-                        const double shx = ox * sd.h[0], shy = oy * sd.h[1];
-                        int zlo = loc[2] - szc, zhi = loc[2] + szc;
-                        if (!(sd.periodic & 4)) {
-                            zlo = max(zlo, 0);
-                            zhi = min(zhi, sd.cdim[2] - 1);
+                    // Chunks of the candidate row.  A bit per candidate marks
+                    // the starts of its cells, so that a lane finds the cell
+                    // of its candidate by counting bits; kPassBatch passes of
+                    // 64 candidates are loaded together (four spill 31
+                    // registers; with velocities two cost a wave per SIMD:
+                    // 200,000 DPD particles 284 us a step with one, 340 with two).  (Staging cell column
+                    // after column, each with its own chain of loads and its
+                    // scalar bookkeeping, was half of the time of sparse
+                    // systems.)
+                    constexpr int kPassBatch = DPD || FLUX ? 1 : 2;
+                    for (int cb = 0; cb < total; cb += chunk) {
+                        const int count = min(chunk, total - cb);
+                        for (int w = tfirst; w < chunk / 32; w += tstep_of) s_mark[w] = 0u;
+                        sync();
+                        int before = 0;   // cells that start before the chunk
+                        for (int k0 = 0; k0 < nseg; k0 += kWave) {
+                            const int rel = k0 + lane < nseg ? s_seg[3 * (k0 + lane)] - cb : count;
+                            if (rel >= 0 && rel < count) atomicOr(&s_mark[rel >> 5], 1u << (rel & 31));
+                            before += __popcll(__ballot(rel < 0));
                         }
-                        // The column's cells are contiguous in memory unless the z range
-                        // wraps around the periodic boundary; then it is two runs.
-                        const bool wrap_lo = zlo < 0, wrap_hi = zhi >= sd.cdim[2];
-                        const int nruns = (wrap_lo || wrap_hi) ? 2 : 1;
-                        for (int run = 0; run < nruns; run++) {
-                            int zf, nzc, oz0;
-                            if (!wrap_lo && !wrap_hi) {
-                                zf = zlo; nzc = zhi - zlo + 1; oz0 = zlo - loc[2];
-                            } else if (wrap_lo) {
-                                if (run == 0) { zf = zlo + sd.cdim[2]; nzc = -zlo; oz0 = -szc; }
-                                else { zf = 0; nzc = zhi + 1; oz0 = -loc[2]; }
-                            } else {
-                                if (run == 0) { zf = zlo; nzc = sd.cdim[2] - zlo; oz0 = -szc; }
-                                else { zf = 0; nzc = zhi - sd.cdim[2] + 1; oz0 = sd.cdim[2] - loc[2]; }
+                        sync();
+                        // lane l holds word l of the marks and the marks before it
+                        const int word = lane < chunk / 32 ? static_cast<int>(s_mark[lane]) : 0;
+                        int marks = __popc(static_cast<unsigned>(word));
+#pragma unroll
+                        for (int o = 1; o < kWave; o <<= 1) {
+                            const int y = __shfl_up(marks, o);
+                            if (lane >= o) marks += y;
+                        }
+                        marks += before - 1 - __popc(static_cast<unsigned>(word));
+                        const int passes = (count + kWave - 1) / kWave;
+                        const int pstep = share ? kNbWaves : 1;
+                        for (int p0 = share ? wid : 0; p0 < passes; p0 += pstep * kPassBatch) {
+                            int sjv[kPassBatch], codev[kPassBatch];
+                            v4 pv[kPassBatch];
+                            int2 mv[kPassBatch];
+                            v4 velv[DPD ? kPassBatch : 1];
+#pragma unroll
+                            for (int u = 0; u < kPassBatch; u++) {
+                                const int p = min(p0 + u * pstep, passes - 1);
+                                const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_readlane(word, 2 * p));
+                                const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_readlane(word, 2 * p + 1));
+                                const int rel = p * kWave + lane;
+                                // the last start at or before this candidate
+                                const int own = static_cast<int>((lane < 32 ? lo >> lane : hi >> (lane - 32)) & 1u);
+                                const int rank = __builtin_amdgcn_readlane(marks, 2 * p) +
+                                                 static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u))) + own;
+                                const int *e = s_seg + 3 * rank;
+                                sjv[u] = e[1] + cb + (rel < count ? rel : 0);
+                                if (rel >= count) sjv[u] = si;   // past the end: any slot
+                                codev[u] = e[2];
                             }
-                            // first slot of each cell of the run (cells 1 .. nzc-1 set oz)
-                            int bnd[2 * kMaxSpanZ + 1];
 #pragma unroll
-                            for (int m = 0; m < 2 * kMaxSpanZ + 1; m++)
-                                bnd[m] = m <= nzc ? P.start[colbase + zf + m] : 0x7fffffff;
-                            int ja = bnd[0];
-                            const int jend = P.start[colbase + zf + nzc];
-                            while (ja < jend) {
-                                const int take = min(jend - ja, chunk - nstaged);
-                                for (int t = lane; t < take; t += kWave) {
-                                    const int sj = ja + t;
-                                    int oz = oz0;
+                            for (int u = 0; u < kPassBatch; u++) {
+                                pv[u] = P.A.pos[sjv[u]];
+                                mv[u] = *reinterpret_cast<const int2 *>(&P.A.meta[sjv[u]]);
+                                if (DPD) velv[u] = P.A.vel[sjv[u]];
+                            }
 #pragma unroll
-                                    for (int m = 1; m < 2 * kMaxSpanZ + 1; m++) {
-                                        if (m >= nzc) break;
-                                        oz += sj >= bnd[m] ? 1 : 0;
-                                    }
-                                    v4 p = P.A.pos[sj];
-                                    const int2 mj = *reinterpret_cast<const int2 *>(&P.A.meta[sj]);
-                                    if (EXT) s_rad[nstaged + t] = p.w;
-                                    p.x = real(static_cast<double>(p.x) + shx);
-                                    p.y = real(static_cast<double>(p.y) + shy);
-                                    p.z = real(static_cast<double>(p.z) + oz * sd.h[2]);
-                                    p.w = as_real_bits(type_column<v4>(mj.x & 0xffff), real(0));
-                                    s_pos[nstaged + t] = p;
-                                    if (kStageIds) s_id[nstaged + t] = mj.y;
-                                    if (kGuarded) s_slot[nstaged + t] = sj;
-                                    if (DPD) s_vel[nstaged + t] = P.A.vel[sj];
-                                    if (FLUX)
-                                        for (int k = 0; k < S; k++)
-                                            s_sp[(nstaged + t) * S + k] = P.A.sp[(size_t)k * P.np + sj];
-                                }
-                                if (si >= ja && si < ja + take) self_k = nstaged + si - ja;
-                                nstaged += take;
-                                ja += take;
-                                if (nstaged == chunk) {
-                                    wave_sync();
-                                    process(nstaged);
-                                    wave_sync();
-                                    nstaged = 0;
-                                    self_k = -1;
-                                }
+                            for (int u = 0; u < kPassBatch; u++) {
+                                const int rel = (p0 + u * pstep) * kWave + lane;
+                                if (rel >= count) continue;
+                                const int code = codev[u];
+                                v4 p = pv[u];
+                                if (EXT) s_rad[rel] = p.w;
+                                p.x = real(static_cast<double>(p.x) + (code / (kCodeSide * kCodeSide) - kMaxSpan) * sd.h[0]);
+                                p.y = real(static_cast<double>(p.y) + (code / kCodeSide % kCodeSide - kMaxSpan) * sd.h[1]);
+                                p.z = real(static_cast<double>(p.z) + (code % kCodeSide - kMaxSpan) * sd.h[2]);
+                                p.w = as_real_bits(type_column<v4>(mv[u].x & 0xffff), real(0));
+                                s_pos[rel] = p;
+                                if (kStageIds) s_id[rel] = mv[u].y;
+                                if (kGuarded) s_slot[rel] = sjv[u];
+                                if (DPD) s_vel[rel] = velv[u];
+                                if (FLUX)
+                                    for (int k = 0; k < S; k++) s_sp[rel * S + k] = P.A.sp[(size_t)k * P.np + sjv[u]];
                             }
                         }
+                        sync();
+                        self_k = self_base + si - cb;
+                        if (self_k < 0 || self_k >= count) self_k = -1;
+                        process(count);
+                        sync();
                     }
                 }
-                if (nstaged > 0) {
+                if (BUILD && nstaged > 0) {
                     wave_sync();
-                    if (BUILD) self_k = active ? s_self[il] : -1;
+                    self_k = active ? s_self[il] : -1;
                     process(nstaged);
                     wave_sync();
                 }
@@ -982,6 +1056,7 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                     }
                     wave_sync();
                 }
+                if (share) __syncthreads();   // the region is staged anew next
                 if (active && sl == 0) {
                     v4 fo;
                     fo.x = fx;
@@ -1057,12 +1132,12 @@ static int variant_key(const DeviceEnsemble *E) {
     return (E->has_dpd ? 4 : 0) | (E->has_flux ? 2 : 0) | (E->has_ext ? 1 : 0);
 }
 
-template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_nt, int max_coef) {
+template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_nt, int max_coef, int max_stencil) {
     const size_t cbytes = static_cast<size_t>(max_coef) * sizeof(real);
     E->coef_lds_bytes = (cbytes > 0 && cbytes <= static_cast<size_t>(kCoefLdsMax)) ? static_cast<int>(cbytes) : 0;
     const int max_chunk = 512;
     E->nb = nb_layout<real>(max_nt, E->coef_lds_bytes > 0 ? max_coef : 0, E->S, E->has_dpd, E->has_flux,
-                            E->has_ext, max_chunk);
+                            E->has_ext, max_chunk, false, max_stencil, &E->nbs);
     // resident workgroups of the variant that runs every step (no energies)
     const void *fn = pick_nonbond<real>(variant_key(E), E->coef_lds_bytes > 0, false);
     int per_cu = 0;
@@ -1099,7 +1174,7 @@ template <typename real> int run_list_build(DeviceEnsemble *E, const KP<real> &P
     KP<real> Q = P;
     Q.nb = E->nbb;
     void *args[] = {&Q};
-    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(&k_list_build<real>), dim3(E->nonbond_grid()),
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(&k_list_build<real>), dim3(E->build_grid()),
                                          dim3(kNbThreads), args, E->nbb.total, E->stream);
     if (e != hipSuccess) return set_error(TFG_E_DEVICE, std::string("list build: ") + hipGetErrorString(e));
     return launch_error("list build");
@@ -1647,7 +1722,7 @@ template int run_list_build<float>(DeviceEnsemble *, const KP<float> &);
 template int run_list_build<double>(DeviceEnsemble *, const KP<double> &);
 template int run_nonbond<float>(DeviceEnsemble *, const KP<float> &);
 template int run_nonbond<double>(DeviceEnsemble *, const KP<double> &);
-template int nonbond_setup<float>(DeviceEnsemble *, int, int);
-template int nonbond_setup<double>(DeviceEnsemble *, int, int);
+template int nonbond_setup<float>(DeviceEnsemble *, int, int, int);
+template int nonbond_setup<double>(DeviceEnsemble *, int, int, int);
 
 }  // namespace tfg
