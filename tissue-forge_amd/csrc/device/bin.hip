@@ -5,8 +5,8 @@
 // 13-direction sorts of runner_dosort, tf_runner_dosort.cpp:64-126) with:
 //   scan      exclusive prefix of the per-cell counts (from the advance pass)
 //   scatter   slot reservation per run of equal cell ids in a wave
-//   order     particles of each cell ordered by particle id (canonical order)
-//   permute   gather of every particle array from buffer B into buffer A
+//   order     particles of each cell ordered by particle id (canonical order),
+//             and every particle array gathered from buffer B into buffer A
 // The cell id of every particle is computed by the advance pass with the
 // reference's incremental rule; binning only reorders.
 //
@@ -27,6 +27,19 @@ constexpr int kScanTile = kScanBlock * kScanPer;
 // A binning kernel does nothing when the step keeps its order (gate is the
 // rebuild flag in list mode, null otherwise) or the ensemble is halted.
 __device__ inline bool bin_skip(const int *gate, const int *halt) { return (gate && *gate == 0) || *halt != 0; }
+
+// The same at the start of a step without lists, where the first kernel of the
+// binning also counts the step (a launch of its own took 4 us, of 95 us at
+// 30,000 particles): a failure of the last update (err[1]) becomes a halt, and
+// a halted ensemble does not count the step.  step: null in any other binning.
+// Every block comes to the same answer, whether or not it sees the halt that
+// block 0 writes.
+__device__ inline bool begin_skip(const int *gate, long long *step, int *err) {
+    if (!step) return bin_skip(gate, err);
+    const bool halted = err[0] != 0 || err[1] != 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && !tick_halted(err)) *step += 1;
+    return halted;
+}
 
 __device__ inline int block_exclusive_scan(int v, int *s) {
     // 1024 threads: wave-level inclusive scan with shuffles, then wave totals.
@@ -53,8 +66,8 @@ __device__ inline int block_exclusive_scan(int v, int *s) {
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int *cnt, int *bsum, int n, const int *gate,
-                                                           const int *halt) {
-    if (bin_skip(gate, halt)) return;
+                                                           long long *step, int *err) {
+    if (begin_skip(gate, step, err)) return;
     __shared__ int s[16];
     const int base = blockIdx.x * kScanTile + threadIdx.x * kScanPer;
     int v = 0;
@@ -102,35 +115,45 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const int *cnt, const
     if (blockIdx.x == 0 && threadIdx.x == 0) start[n] = bsum[nb];
 }
 
-// The whole scan in one block, tile after tile with a carry: for grids of a
-// few tiles, where the three-kernel scan would be mostly launches.
-constexpr int kScanSingleMax = 4 * kScanTile;
+// The whole scan in one block of PER counts per thread, for grids of up to
+// 16,384 cells, where the three-kernel scan would be mostly launches.  Bound by
+// the latency of one pass of loads and the block scan: the counts are read
+// four at a time, all at once (tile after tile with a carry 8.8 us at 15,625
+// cells, so 4.8).
+constexpr int kScanSingleMax = 16 * kScanBlock;
+template <int PER>
 __global__ __launch_bounds__(kScanBlock) void k_scan_single(const int *cnt, int *start, int n, const int *gate,
-                                                           const int *halt) {
-    if (bin_skip(gate, halt)) return;
+                                                           long long *step, int *err) {
+    if (begin_skip(gate, step, err)) return;
     __shared__ int s[16];
-    __shared__ int tot;
-    int carry = 0;
-    for (int t0 = 0; t0 < n; t0 += kScanTile) {
-        const int base = t0 + threadIdx.x * kScanPer;
-        int c[kScanPer];
-        int v = 0;
-        for (int k = 0; k < kScanPer; k++) {
-            c[k] = base + k < n ? cnt[base + k] : 0;
-            v += c[k];
-        }
-        const int ex = block_exclusive_scan(v, s);
-        int run = carry + ex;
-        for (int k = 0; k < kScanPer; k++) {
-            if (base + k < n) start[base + k] = run;
-            run += c[k];
-        }
-        if (threadIdx.x == kScanBlock - 1) tot = ex + v;
-        __syncthreads();
-        carry += tot;
-        __syncthreads();
+    const int base = threadIdx.x * PER;
+    int4 c[PER / 4];
+    int v = 0;
+#pragma unroll
+    for (int k = 0; k < PER / 4; k++) {
+        const int at = base + 4 * k;
+        if (at + 3 < n)
+            c[k] = *reinterpret_cast<const int4 *>(cnt + at);
+        else
+            c[k] = make_int4(at < n ? cnt[at] : 0, at + 1 < n ? cnt[at + 1] : 0, at + 2 < n ? cnt[at + 2] : 0, 0);
     }
-    if (threadIdx.x == 0) start[n] = carry;
+#pragma unroll
+    for (int k = 0; k < PER / 4; k++) v += c[k].x + c[k].y + c[k].z + c[k].w;
+    int run = block_exclusive_scan(v, s);
+#pragma unroll
+    for (int k = 0; k < PER / 4; k++) {
+        const int at = base + 4 * k;
+        const int4 o = make_int4(run, run + c[k].x, run + c[k].x + c[k].y, run + c[k].x + c[k].y + c[k].z);
+        run = o.w + c[k].w;
+        if (at + 3 < n) {
+            *reinterpret_cast<int4 *>(start + at) = o;
+        } else {
+            if (at < n) start[at] = o.x;
+            if (at + 1 < n) start[at + 1] = o.y;
+            if (at + 2 < n) start[at + 2] = o.z;
+        }
+    }
+    if (threadIdx.x == kScanBlock - 1) start[n] = run;
 }
 
 // The slots of every bond's and angle's particles (and its potential), after
@@ -181,29 +204,87 @@ __global__ void k_scatter(const int4 *meta, const int *start, int *fill, int2 *t
         const int key = m.z;
         int head, len;
         wave_runs(key, valid, lane, &head, &len);
+        const int first = valid ? start[key] : 0;   // (in flight with the atomic)
         int r = 0;
         if (valid && head == lane) r = atomicAdd(&fill[key], len);
         const int rb = __shfl(r, head);
-        if (valid) tmp[start[key] + rb + (lane - head)] = make_int2(m.y, i);
+        if (valid) tmp[first + rb + (lane - head)] = make_int2(m.y, i);
     }
 }
 
-// Orders each cell by particle id and writes the gather permutation; clears
-// the counters for the next step.  Cells of up to 16 particles are ranked in
-// 16-lane groups with shuffles, four cells per wave; larger cells use the
-// whole wave.
-__global__ __launch_bounds__(64) void k_cellorder(const int *start, const int2 *tmp, int *perm, int *cnt,
-                                                  int *fill, int ncells, const int *gate, const int *halt) {
-    if (bin_skip(gate, halt)) return;
+// Particle src of buffer B into slot dst of buffer A.  Every load comes before
+// the first store: written array by array the stores, which may alias as far
+// as the compiler knows, put the loads' latencies one after the other.
+template <typename real> __device__ inline void move_particle(const KP<real> &P, int src, int dst) {
+    using v4 = typename V<real>::v4;
+    constexpr int kSp = 4;   // species per batch of loads
+    const v4 x = P.B.pos[src], v = P.B.vel[src];
+    const int4 m = P.B.meta[src];
+    const real im = P.B.imass[src];
+    if (P.A.p0) {   // Runge-Kutta stage state
+        const v4 p0 = P.B.p0[src], v0 = P.B.v0[src], sx = P.B.sx[src], sv = P.B.sv[src], vk = P.B.vk[src];
+        P.A.p0[dst] = p0;
+        P.A.v0[dst] = v0;
+        P.A.sx[dst] = sx;
+        P.A.sv[dst] = sv;
+        P.A.vk[dst] = vk;
+    }
+    for (int k0 = 0; k0 < P.S; k0 += kSp) {
+        real c[kSp], q[kSp];
+#pragma unroll
+        for (int u = 0; u < kSp; u++)
+            if (k0 + u < P.S) {
+                c[u] = P.B.sp[(size_t)(k0 + u) * P.np + src];
+                q[u] = P.B.q[(size_t)(k0 + u) * P.np + src];
+            }
+#pragma unroll
+        for (int u = 0; u < kSp; u++)
+            if (k0 + u < P.S) {
+                P.A.sp[(size_t)(k0 + u) * P.np + dst] = c[u];
+                P.A.q[(size_t)(k0 + u) * P.np + dst] = q[u];
+            }
+    }
+    P.A.pos[dst] = x;
+    P.A.vel[dst] = v;
+    P.A.meta[dst] = m;
+    P.A.imass[dst] = im;
+    P.slot_of[m.y] = dst;
+    if (P.list_mode) {   // the state the new lists are built from
+        P.x0[dst] = x;
+        P.cid0[dst] = m.z;
+        v4 xb = x;
+        xb.w = as_real_bits(type_column<v4>(m.x & 0xffff), real(0));
+        P.xb[dst] = xb;
+    }
+}
+
+// Orders each cell by particle id and moves its particles from B to their
+// slots in A; clears the counters for the next step.  Cells of up to 16
+// particles are ranked in 16-lane groups with shuffles, four cells per wave;
+// larger cells use the whole wave.  Systems that keep their lists keep their
+// order (only their counters are cleared).
+//
+// Bound by latencies: cell bounds, the cell's entries, the particles.  A
+// permutation written here and gathered by a kernel of its own cost a launch
+// and its loads one after the other (move_particle); both kernels then, this
+// one now: 30,000 particles 17.5, 8.6 us, 24,000 DPD 14.8, 5.5,
+// 100,000 22.7, 7.5, 64,000 Runge-Kutta 25.3, 12.3.
+template <typename real>
+__global__ __launch_bounds__(64) void k_order(KP<real> P, const int *gate) {
+    if (bin_skip(gate, P.err)) return;
     __shared__ int keys[2048];
+    const int *start = P.start;
+    const int2 *tmp = P.tmp;
     const int lane = threadIdx.x;
     const int g = lane >> 4, e = lane & 15;
-    for (int c0 = blockIdx.x * 4; c0 < ncells; c0 += gridDim.x * 4) {
+    for (int c0 = blockIdx.x * 4; c0 < P.ncells; c0 += gridDim.x * 4) {
         const int c = c0 + g;
         int s0 = 0, n = 0;
-        if (c < ncells) {
+        bool keeps = false;
+        if (c < P.ncells) {
             s0 = start[c];
             n = start[c + 1] - s0;
+            keeps = P.list_mode && P.sflags[P.nsys + P.cell_sys[c]] == 0;
         }
         const bool small = n <= 16;
         int2 me = make_int2(0x7fffffff, -1);
@@ -213,17 +294,16 @@ __global__ __launch_bounds__(64) void k_cellorder(const int *start, const int2 *
             const int k = __shfl(me.x, (g << 4) + o);
             rank += (o < n) && (k < me.x);
         }
-        if (small && e < n) perm[s0 + rank] = me.y;
-        if (c < ncells && e == 0) {
-            cnt[c] = 0;
-            fill[c] = 0;
+        if (c < P.ncells && e == 0) {
+            P.cnt[c] = 0;
+            P.fill[c] = 0;
         }
-        unsigned long long big = __ballot(c < ncells && !small && e == 0);
+        if (small && e < n && !keeps) move_particle<real>(P, me.y, s0 + rank);
+        unsigned long long big = __ballot(c < P.ncells && !small && !keeps && e == 0);
         while (big) {
             const int gl = __builtin_ctzll(big) >> 4;
             big &= big - 1;
-            const int cb = c0 + gl;
-            const int sb = start[cb], nb = start[cb + 1] - sb;
+            const int sb = __shfl(s0, gl << 4), nb = __shfl(n, gl << 4);
             const bool lds = nb <= 2048 - 8;
             __syncthreads();
             if (lds) {
@@ -247,7 +327,7 @@ __global__ __launch_bounds__(64) void k_cellorder(const int *start, const int2 *
                 } else {
                     for (int o = 0; o < nb; o++) rk += tmp[sb + o].x < mine.x;
                 }
-                perm[sb + rk] = mine.y;
+                move_particle<real>(P, mine.y, sb + rk);
             }
         }
     }
@@ -282,52 +362,15 @@ template <typename real> int run_sync(DeviceEnsemble *E, const KP<real> &P, bool
 template int run_sync<float>(DeviceEnsemble *, const KP<float> &, bool);
 template int run_sync<double>(DeviceEnsemble *, const KP<double> &, bool);
 
-template <typename real>
-__global__ void k_permute(KP<real> P) {
-    using v4 = typename V<real>::v4;
-    const int S = P.S;
-    if (P.err[0] != 0) return;   // halted
-    if (P.list_mode && P.lflags[0] == 0) return;   // A holds the state of systems that keep their lists
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < P.np; i += gridDim.x * blockDim.x) {
-        // slot i belongs to the system of the particle buffer B holds there;
-        // systems that keep their lists keep their order
-        if (P.list_mode && P.sflags[P.nsys + P.cell_sys[P.B.meta[i].z]] == 0) continue;
-        const int src = P.perm[i];
-        P.A.pos[i] = P.B.pos[src];
-        P.A.vel[i] = P.B.vel[src];
-        const int4 m = P.B.meta[src];
-        P.A.meta[i] = m;
-        P.A.imass[i] = P.B.imass[src];
-        for (int k = 0; k < S; k++) {
-            P.A.sp[(size_t)k * P.np + i] = P.B.sp[(size_t)k * P.np + src];
-            P.A.q[(size_t)k * P.np + i] = P.B.q[(size_t)k * P.np + src];
-        }
-        if (P.list_mode) {   // the state the new lists are built from
-            v4 p = P.A.pos[i];
-            P.x0[i] = p;
-            P.cid0[i] = m.z;
-            p.w = as_real_bits(type_column<v4>(m.x & 0xffff), real(0));
-            P.xb[i] = p;
-        }
-        if (P.A.p0) {   // Runge-Kutta stage state
-            P.A.p0[i] = P.B.p0[src];
-            P.A.v0[i] = P.B.v0[src];
-            P.A.sx[i] = P.B.sx[src];
-            P.A.sv[i] = P.B.sv[src];
-            P.A.vk[i] = P.B.vk[src];
-        }
-        P.slot_of[m.y] = i;
-    }
-}
-
 int run_count(DeviceEnsemble *E) {
     hipLaunchKernelGGL(k_count, dim3(E->stream_grid()), dim3(E->shape.stream_threads), 0, E->stream, E->meta[1],
                        E->cnt, E->np, nullptr, E->d_err);
     return launch_error("count");
 }
 
-template <typename real> int run_bin(DeviceEnsemble *E, const KP<real> &P) {
+template <typename real> int run_bin(DeviceEnsemble *E, const KP<real> &P, bool begin) {
     hipStream_t s = E->stream;
+    long long *step = begin ? E->d_step : nullptr;
     const int nb = (E->ncells + kScanTile - 1) / kScanTile;
     const int g = E->stream_grid(), t = E->shape.stream_threads;
     const int *gate = E->list_mode ? E->d_lflags : nullptr;
@@ -335,10 +378,15 @@ template <typename real> int run_bin(DeviceEnsemble *E, const KP<real> &P) {
     if ((rc = run_sync<real>(E, P, false)) != TFG_OK) return rc;   // a rebuild bins from B
     if (E->list_mode)
         hipLaunchKernelGGL(k_count, dim3(g), dim3(t), 0, s, E->meta[1], E->cnt, E->np, gate, E->d_err);
-    if (E->ncells <= kScanSingleMax) {
-        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanBlock), 0, s, E->cnt, E->start, E->ncells, gate, E->d_err);
+    if (E->ncells <= 4 * kScanBlock) {
+        hipLaunchKernelGGL(k_scan_single<4>, dim3(1), dim3(kScanBlock), 0, s, E->cnt, E->start, E->ncells, gate, step,
+                           E->d_err);
+    } else if (E->ncells <= kScanSingleMax) {
+        hipLaunchKernelGGL(k_scan_single<16>, dim3(1), dim3(kScanBlock), 0, s, E->cnt, E->start, E->ncells, gate, step,
+                           E->d_err);
     } else {
-        hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanBlock), 0, s, E->cnt, E->bsum, E->ncells, gate, E->d_err);
+        hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanBlock), 0, s, E->cnt, E->bsum, E->ncells, gate, step,
+                           E->d_err);
         hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanBlock), 0, s, E->bsum, nb, gate, E->d_err);
         hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, s, E->cnt, E->bsum, E->start, E->ncells, nb,
                            gate, E->d_err);
@@ -347,16 +395,14 @@ template <typename real> int run_bin(DeviceEnsemble *E, const KP<real> &P) {
     // grid-stride over groups of four cells; a modest grid keeps the launch
     // cheap in the list steps that skip it
     const int oc = std::min((E->ncells + 3) / 4, 8192);
-    hipLaunchKernelGGL(k_cellorder, dim3(oc), dim3(64), 0, s, E->start, E->tmp, E->perm, E->cnt, E->fill, E->ncells,
-                       gate, E->d_err);
-    hipLaunchKernelGGL(k_permute<real>, dim3(g), dim3(t), 0, s, P);
+    hipLaunchKernelGGL(k_order<real>, dim3(oc), dim3(64), 0, s, P, gate);
     if (E->nbonds + E->nangles > 0)
         hipLaunchKernelGGL(k_term_slots, dim3(g), dim3(t), 0, s, E->d_bonds, E->d_angles, E->slot_of, E->d_bslot,
                            E->d_aslot, E->nbonds, E->nangles, gate, E->d_err);
     return launch_error("binning");
 }
 
-template int run_bin<float>(DeviceEnsemble *, const KP<float> &);
-template int run_bin<double>(DeviceEnsemble *, const KP<double> &);
+template int run_bin<float>(DeviceEnsemble *, const KP<float> &, bool);
+template int run_bin<double>(DeviceEnsemble *, const KP<double> &, bool);
 
 }  // namespace tfg

@@ -197,7 +197,7 @@ template <typename real> struct KP {
     PArrays<real> A, B;
     typename V<real>::v4 *force;   // force + number density, A order
     int *slot_of;
-    int *cnt, *fill, *start, *perm, *bsum;
+    int *cnt, *fill, *start, *bsum;
     int2 *tmp;
     double *e_part;   // energy partials
     double *e_nb, *e_vir, *e_kin, *e_bond, *e_ang;
@@ -308,6 +308,13 @@ __device__ inline void wave_runs(int key, bool valid, int lane, int *head, int *
     const unsigned long long after = lane == 63 ? 0ull : (heads >> (lane + 1));
     const int next = after ? lane + 1 + __builtin_ctzll(after) : nvalid;
     *len = next - lane;
+}
+
+// Start of a step: a failure of the last update (err[1]) becomes a halt;
+// a halted ensemble does not count the step.
+__device__ inline bool tick_halted(int *err) {
+    if (err[1] != 0) err[0] |= kHaltTooFast;
+    return err[0] != 0;
 }
 
 }  // namespace tfg

@@ -112,7 +112,7 @@ struct DeviceEnsemble {
     void *rk[2][5] = {{nullptr}};   // Runge-Kutta p0, v0, sx, sv, vk per buffer
     int4 *meta[2] = {nullptr, nullptr};
     void *force = nullptr;
-    int *slot_of = nullptr, *cnt = nullptr, *fill = nullptr, *start = nullptr, *perm = nullptr, *bsum = nullptr;
+    int *slot_of = nullptr, *cnt = nullptr, *fill = nullptr, *start = nullptr, *bsum = nullptr;
     int2 *tmp = nullptr;
     double *e_part = nullptr, *e_nb = nullptr, *e_vir = nullptr, *e_kin = nullptr, *e_bond = nullptr,
            *e_ang = nullptr;
@@ -197,9 +197,10 @@ int ensemble_force_arena(Engine *e, int precision, void *arena, size_t cap, doub
 int read_into_engine(DeviceEnsemble *E, int s);
 int restore_kept(DeviceEnsemble *E);
 
-// Binning: scan of the cell counts, placement, per-cell order, permutation
-// of buffer B into buffer A.  Cell counts come from the previous advance.
-template <typename real> int run_bin(DeviceEnsemble *E, const KP<real> &P);
+// Binning: scan of the cell counts, placement, per-cell order and move of
+// buffer B into buffer A.  Cell counts come from the previous advance.  begin:
+// the first kernel of a step without lists, which also counts the step.
+template <typename real> int run_bin(DeviceEnsemble *E, const KP<real> &P, bool begin);
 template <typename real> int run_sync(DeviceEnsemble *E, const KP<real> &P, bool force);
 // Counts particles per cell from buffer B (after an upload).
 int run_count(DeviceEnsemble *E);

@@ -62,7 +62,6 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy) {
     P.cnt = E->cnt;
     P.fill = E->fill;
     P.start = E->start;
-    P.perm = E->perm;
     P.bsum = E->bsum;
     P.tmp = E->tmp;
     P.e_part = E->e_part;
@@ -108,17 +107,6 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy) {
     P.sflags = E->d_sflags;
     P.nsys = E->nsys;
     return P;
-}
-
-// Start of a step: a failure of the last update (err[1]) becomes a halt;
-// a halted ensemble does not count the step.
-__device__ inline bool tick_halted(int *err) {
-    if (err[1] != 0) err[0] |= kHaltTooFast;
-    return err[0] != 0;
-}
-
-__global__ void k_tick(long long *step, int *err) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && !tick_halted(err)) *step += 1;
 }
 
 // List mode: a system rebuilds in this step when the last advance asked for
@@ -241,7 +229,7 @@ template <typename real> static int enqueue_step(DeviceEnsemble *E, bool energy,
         hipLaunchKernelGGL(k_tick_list, dim3(1), dim3(256), 0, E->stream, E->d_step, E->d_lflags, E->d_sflags, E->nsys,
                            E->d_err);
         if (ev) TFG_HIP(hipEventRecord(ev[0], E->stream));
-        if ((rc = run_bin<real>(E, Pe)) != TFG_OK) return rc;
+        if ((rc = run_bin<real>(E, Pe, false)) != TFG_OK) return rc;
         if (ev) TFG_HIP(hipEventRecord(ev[1], E->stream));
         if ((rc = run_list_build<real>(E, Pe)) != TFG_OK || (rc = run_near<real>(E, Pe)) != TFG_OK) return rc;
         if (ev) TFG_HIP(hipEventRecord(ev[2], E->stream));
@@ -258,14 +246,13 @@ template <typename real> static int enqueue_step(DeviceEnsemble *E, bool energy,
         if (energy && (rc = run_energy<real>(E, Pe)) != TFG_OK) return rc;
         return TFG_OK;
     }
-    hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, E->stream, E->d_step, E->d_err);
     const bool rk4 = E->integrator == INTEG_RUNGE_KUTTA_4;
     const int rounds = rk4 ? 4 : 1;
     for (int st = 0; st < rounds; st++) {
         const bool last = st == rounds - 1;
         const KP<real> &Q = last ? Pe : P;
         if (ev && last) TFG_HIP(hipEventRecord(ev[0], E->stream));
-        if ((rc = run_bin<real>(E, Q)) != TFG_OK) return rc;
+        if ((rc = run_bin<real>(E, Q, st == 0)) != TFG_OK) return rc;   // the first counts the step
         if (ev && last) TFG_HIP(hipEventRecord(ev[1], E->stream));
         if (ev && last) TFG_HIP(hipEventRecord(ev[2], E->stream));   // no list build
         // The sub-step pair pass is the full pair kernel; only its pending
@@ -746,7 +733,6 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     ALLOC(E->fill, int, nc);
     ALLOC(E->start, int, nc + 1);
     ALLOC(E->bsum, int, nb_scan + 1);
-    ALLOC(E->perm, int, np);
     ALLOC(E->tmp, int2, np);
     ALLOC(E->e_nb, double, np);
     ALLOC(E->e_vir, double, np);
@@ -1084,7 +1070,7 @@ template <typename real> static int force_t(DeviceEnsemble *E) {
     if (E->list_mode)
         hipLaunchKernelGGL(k_list_rebin, dim3(1), dim3(256), 0, E->stream, E->d_lflags, E->d_sflags, E->nsys);
     if (timed) TFG_HIP(hipEventRecord(E->ev[0], E->stream));
-    if ((rc = run_bin<real>(E, P)) != TFG_OK) return rc;
+    if ((rc = run_bin<real>(E, P, false)) != TFG_OK) return rc;
     if (timed) TFG_HIP(hipEventRecord(E->ev[1], E->stream));
     // list mode: the lists of the new order (timed for the autotuner, which
     // tunes the build's grid); the next step rebuilds again
