@@ -697,19 +697,33 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                     }
                 };
 
-                // Candidates [0, count) of the staged list.
+                // Candidates [0, count) of the staged list, in rounds of up to
+                // 128 per lane.  The slices of a particle take its candidates
+                // in turn: candidates lie cell by cell, and with a run of them
+                // per slice one slice had a near cell's pairs, all in range,
+                // and the others waited.  Microseconds a step with runs, in
+                // turn: 30,000 particles 92, 76, 200,000 270, 207, radii
+                // 100,000 140, 125, mixture 1M 698, 631, DPD 200,000 267, 260.
+                // The build takes runs, for the order of its lists.
                 auto process = [&](int count) {
-                    const int cap = slices > 1 ? 127 : 128;
+                    const int cap = BUILD && slices > 1 ? 127 : 128;
+                    const int step = BUILD ? 1 : slices;
                     for (int rb = 0; rb < count; rb += cap * slices) {
                         const int rcount = min(count - rb, cap * slices);
                         int per = (rcount + slices - 1) / slices;
-                        if (slices > 1) per |= 1;   // odd stride: slices start on different banks
-                        const int kb = rb + sl * per;
-                        const int my = active ? max(0, min(per, rb + rcount - kb)) : 0;
+                        if (BUILD && slices > 1) per |= 1;   // odd stride: slices start on different banks
+                        const int kb = BUILD ? rb + sl * per : rb + sl;
+                        const int my = !active ? 0
+                                       : BUILD ? max(0, min(per, rb + rcount - kb))
+                                               : (rcount - sl + slices - 1) / slices;
                         const v4 *sp4 = s_pos + kb;
+                        const int klim = max(count - 1, 0);
                         unsigned long long m0 = 0, m1 = 0;
-#pragma unroll
-                        for (int blk = 0; blk < 8; blk++) {
+                        // (written out, the blocks cost FP32 tables 2 to 5%;
+                        // as a loop they cost DPD a wave per SIMD, 16%)
+                        constexpr int kBlocks = BUILD || DPD ? 8 : 1;
+#pragma unroll kBlocks
+                        for (int blk = 0; blk * 16 < (kBlocks == 8 ? 128 : per); blk++) {
                             if (blk * 16 < my) {
                                 unsigned bits = 0;
                                 if constexpr (BUILD) {
@@ -723,10 +737,16 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                                         const real d = fma_of(dz, dz, fma_of(dy, dy, fma_of(dx, dx, -cut2)));
                                         bits = __builtin_amdgcn_alignbit(bits, sign_word(d), 31);
                                     }
-                                } else {
+                                } else if (rb + (blk * 16 + 16) * slices <= lay.chunk + kPad) {
+                                    const v4 *q = sp4 + blk * 16 * slices;
 #pragma unroll
-                                    for (int t = 0; t < 16; t++)
-                                        bits |= static_cast<unsigned>(dist2(pi4, sp4[blk * 16 + t]) <= cut2) << t;
+                                    for (int t = 0; t < 16; t++, q += slices)
+                                        bits |= static_cast<unsigned>(dist2(pi4, *q) <= cut2) << t;
+                                } else {   // the last rows of a full chunk
+                                    for (int t = 0; t < 16 && blk * 16 + t < per; t++)
+                                        bits |= static_cast<unsigned>(
+                                                    dist2(pi4, s_pos[min(kb + (blk * 16 + t) * slices, klim)]) <= cut2)
+                                                << t;
                                 }
                                 const unsigned long long w = static_cast<unsigned long long>(bits) << ((blk & 3) * 16);
                                 if (blk < 4)
@@ -738,7 +758,11 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                         // drop the entries past this lane's block and the particle itself
                         m0 &= my >= 64 ? ~0ull : ((1ull << my) - 1ull);
                         m1 &= my >= 128 ? ~0ull : (my <= 64 ? 0ull : ((1ull << (my - 64)) - 1ull));
-                        const int st = self_k - kb;
+                        int st = self_k - kb;
+                        if constexpr (!BUILD) {
+                            const int at = st / slices;
+                            st = st >= 0 && at * slices == st ? at : -1;
+                        }
                         if (st >= 0 && st < 64) m0 &= ~(1ull << st);
                         if (st >= 64 && st < 128) m1 &= ~(1ull << (st - 64));
                         if constexpr (BUILD) {
@@ -777,18 +801,17 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                         // Evaluate the set bits, two per iteration.  m0 is refilled
                         // from m1 when it runs empty; an empty pick gives ok = false.
                         int base = kb;
-                        const int klim = max(count - 1, 0);
                         while (__any((m0 | m1) != 0ull)) {
                             const bool refill = m0 == 0ull;
                             m0 = refill ? m1 : m0;
                             m1 = refill ? 0ull : m1;
-                            base += refill ? 64 : 0;
+                            base += refill ? 64 * step : 0;
                             int k2[2];
                             bool ok2[2];
 #pragma unroll
                             for (int u = 0; u < 2; u++) {
                                 ok2[u] = m0 != 0ull;
-                                k2[u] = min(base + ctz64_or_31(m0), klim);
+                                k2[u] = min(base + ctz64_or_31(m0) * step, klim);
                                 m0 &= m0 - 1ull;
                             }
                             eval_pair(k2[0], ok2[0], kFreeMode, 0u);
@@ -800,7 +823,7 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                         if (kGuarded && __builtin_expect(__any(deferred), 0)) {
                             deferred = false;
                             for (int t = 0; t < my; t++) {
-                                const int k = kb + t;
+                                const int k = kb + t * step;
                                 const v4 pj = s_pos[k];
                                 const real r2 = dist2(pi4, pj);
                                 if (k == self_k || !(r2 <= cut2)) continue;
