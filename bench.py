@@ -58,7 +58,7 @@ def cell_bytes(precision, dpd_flux=False):
 
 def list_fixed_bytes(precision):
     """Compulsory bytes per particle of the list pair kernel besides its
-    list entries (4 B each): its build-frame position, its type record, its
+    list entries within the cutoff (4 B each): its build-frame position, its type record, its
     entry count and the force written (16 + 16 + 4 + 16 in FP32)."""
     return 52.0 if precision == 0 else 84.0
 
@@ -188,7 +188,10 @@ def time_gpu(tf, W, scene, pots, precision, steps, warmup, skin=0.0, capacity=0)
     if active:
         mean, mx = eng.verlet_entries()
         lists = {"skin": skin, "rebuilds_in_timed_steps": r1 - r0, "capacity": cap, "mean_entries": mean,
-                 "max_entries": mx}
+                 "max_entries": mx,
+                 # of those, the ones within the cutoff (at uniform density):
+                 # what the pair pass cannot do without
+                 "mean_entries_in_cutoff": mean * (scene["cutoff"] / (scene["cutoff"] + skin)) ** 3}
     eng.from_device()
     eng.close()
 
@@ -217,7 +220,7 @@ def roofline(r, n, precision, workload, dpd_flux=False):
     nb_ms = r["kernels"]["nonbond_avg"]
     if r["lists"] is not None:
         kernel = "k_list_force"
-        bytes_pp = list_fixed_bytes(precision) + 4.0 * r["lists"]["mean_entries"]
+        bytes_pp = list_fixed_bytes(precision) + 4.0 * r["lists"]["mean_entries_in_cutoff"]
     else:
         kernel = "k_nonbond"
         bytes_pp = cell_bytes(precision, dpd_flux)

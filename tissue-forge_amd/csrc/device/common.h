@@ -27,9 +27,9 @@ constexpr int kMaxFluxEntries = 64;   // flux entries per system
 // Cell pass of crowded systems (more than kShareMean particles per cell on
 // average at the upload): a cell of more than kShareAbove particles is one
 // workgroup's.  One wave per cell leaves such systems with few waves, each
-// long: 8,000 particles in 216 cells 203 us a step, shared 97; 200,000 in
-// 6,859 cells 365 -> 340.  At 16 per cell sharing leaves a lane too few
-// candidates (1,000,000 particles 0.80 -> 1.53 ms), so those keep the wave.
+// long: 8,000 particles 199 us a step, shared 75; 30,000 190, 77; 200,000
+// 341, 209.  At 16 per cell sharing leaves a lane too few candidates
+// (1,000,000 particles 0.63 ms, shared 0.93), so those keep the wave.
 // The rule looks at the system alone, so that its results do not depend on
 // the ensemble it is in.
 constexpr double kShareMean = 20.0;

@@ -9,18 +9,17 @@
 //
 // Work unit: one wave per cell of i particles (crowded systems: one workgroup
 // per cell, whose waves stage together and take a part of its particles
-// each).  A workgroup of kNbWaves waves owns a contiguous range of cells (workgroups of one XCD own neighbouring
-// ranges, so their stencils meet in that XCD's L2); its waves take the cells
-// of the range in turn and share the pair descriptors and table
-// coefficients of the current system in LDS.  Each wave stages the particles
-// of its stencil in its own LDS region, shifted into the frame of the i cell
-// (the shift is added in FP64 and rounded once).  Lanes are grouped as
-// (i particle, slice of the staged list), with as many slices as fit the 64
-// lanes.  Per round a lane tests a contiguous block of up to 128 candidates
-// into a register bit mask (the test is unrolled with immediate LDS offsets;
-// blocks of different slices start on different LDS banks), then evaluates
-// the set bits, two per iteration.  Slices are combined in a fixed order
-// through LDS: no atomics, results do not depend on scheduling.
+// each).  A workgroup of kNbWaves waves owns a contiguous range of cells
+// (workgroups of one XCD own neighbouring ranges, so their stencils meet in
+// that XCD's L2); its waves take the cells of the range in turn and share the
+// pair descriptors and table coefficients of the current system in LDS.  Each
+// wave stages the particles of its stencil in its own LDS region, shifted into
+// the frame of the i cell (the shift is added in FP64 and rounded once).
+// Lanes are grouped as (i particle, slice of the staged list), with as many
+// slices as fit the 64 lanes.  Per round a lane tests up to 128 candidates, the
+// slices of a particle in turn, into a register bit mask, then evaluates the
+// set bits, two per iteration.  Slices are combined in a fixed order through
+// LDS: no atomics, results do not depend on scheduling.
 //
 // Cutoff guard (FP32): a truncated potential jumps by F(rc) at the cutoff, so
 // a pair whose FP32 distance rounds to the other side of rc than its FP64
