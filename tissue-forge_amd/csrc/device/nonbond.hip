@@ -1102,16 +1102,19 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
 }
 
 // Kernel entries.  The FP32 table-only variants fit 96 VGPRs (5 waves per
-// SIMD) once the compiler is asked for it: the only spill sits outside the
-// cell loops.  DPD, flux and FP64 variants need more registers and run at the
-// occupancy their register count gives.
+// SIMD) with a few spills, which four waves without spills do not make up for
+// (1M particles 629 us a step, 712 with four).  With radius transforms, sums
+// or images 96 VGPRs spill 26, and the radii and ids leave LDS for four waves
+// anyway: 100,000 particles 125 us a step, 110 with four.  DPD, flux and FP64
+// variants need more registers and run at the occupancy their register count
+// gives.
 template <typename real, bool DPD, bool FLUX, bool EXT, bool CLDS, bool ENERGY>
 __global__ __launch_bounds__(kNbThreads) void k_nonbond(KP<real> P) {
     nonbond_body<real, DPD, FLUX, EXT, CLDS, ENERGY>(P);
 }
 
 template <bool EXT, bool CLDS, bool ENERGY>
-__global__ __launch_bounds__(kNbThreads) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_nonbond_f32(KP<float> P) {
+__global__ __launch_bounds__(kNbThreads) __attribute__((amdgpu_waves_per_eu(EXT ? 4 : 5, 8))) void k_nonbond_f32(KP<float> P) {
     nonbond_body<float, false, false, EXT, CLDS, ENERGY>(P);
 }
 
