@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -137,7 +138,10 @@ struct DeviceEnsemble {
     double *status_sums() const { return reinterpret_cast<double *>(status + 1); }
     int light_run = 4;   // light steps between two full ones
 
-    // Readback: a pinned buffer and an event per reading thread.
+    // Readback: a pinned buffer and an event per reading thread.  read_lock is
+    // held over a read: host threads may read several members, or one engine
+    // in several ways, at once, and share the buffers and the kept state.
+    std::mutex read_lock;
     struct ReadSlot {
         unsigned char *ptr = nullptr;
         size_t bytes = 0;

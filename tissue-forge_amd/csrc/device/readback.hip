@@ -160,7 +160,8 @@ struct OnDevice {
 
 // Reads every particle of system s: the wanted fields of each chunk of ids
 // are gathered into a pinned buffer and handed to use(rows, first id, count),
-// which may run on several threads at once for different chunks.
+// which may run on several threads at once for different chunks.  The caller
+// holds read_lock.
 template <typename Use> static int read_system(DeviceEnsemble *E, int s, ReadRows want, Use &&use) {
     const OnDevice on(E->device);
     const int n = E->sys[s].np;
@@ -256,6 +257,7 @@ static void record_rows(Engine &e, const ReadRows &r, int first, int n) {
 }
 
 int read_into_engine(DeviceEnsemble *E, int s) {
+    const std::lock_guard<std::mutex> hold(E->read_lock);
     Engine &e = *E->engines[s];
     double some = 0;
     int some_i = 0;
@@ -308,6 +310,7 @@ static int keep_read(DeviceEnsemble *E, int s) {
 }
 
 int restore_kept(DeviceEnsemble *E) {
+    const std::lock_guard<std::mutex> hold(E->read_lock);
     for (int s = 0; s < static_cast<int>(E->kept_sys.size()); s++) {
         if (!E->kept_sys[s]) continue;
         const OnDevice on(E->device);
@@ -340,6 +343,7 @@ int restore_kept(DeviceEnsemble *E) {
 
 int ensemble_read(DeviceEnsemble *E, int s, const ReadRows &out) {
     if (s < 0 || s >= E->nsys) return set_error(TFG_E_RANGE, "system index out of range");
+    const std::lock_guard<std::mutex> hold(E->read_lock);
     const int rc = read_system(E, s, out, [&](const ReadRows &rows, int first, int n) { copy_rows(rows, out, first, n); });
     return rc == TFG_OK && E->keep_reads ? keep_read(E, s) : rc;
 }
