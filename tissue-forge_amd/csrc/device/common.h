@@ -34,7 +34,8 @@ constexpr int kMaxFluxEntries = 64;   // flux entries per system
 // the ensemble it is in.
 constexpr double kShareMean = 20.0;
 constexpr int kShareAbove = 12;
-constexpr int kMaxSpan = 3;           // cells of cutoff per direction
+constexpr int kMaxSpanZ = 3;          // cells of cutoff along z per direction
+constexpr int kMaxSegCells = 343;     // stencil cells of the cell pass's segment table; larger stencils take several launches
 // FP32 path: pairs within this relative band of the cutoff (or of a table end
 // below it) are decided in FP64 by the pair kernel.
 constexpr double kGuard = 2e-6;
@@ -45,6 +46,7 @@ struct SysDesc {
     int ncells, cell_off, p_off, np, ntypes;
     int share_above;   // cell pass: a cell of more particles is one workgroup's, not one wave's
     int nstencil, stencil_off;   // cells of the neighbour stencil (cell codes)
+    int ybits;                   // their bits of the y offset
     int pot_off, nslots;          // descriptor slots (int2: potential, next slot) from pot_off
     int type_off;
     int sum_all;                  // a sum evaluates every constituent (else up to the first in range)
@@ -103,12 +105,19 @@ constexpr int kNearLife = 4, kNearRetry = 16, kNearRetryMost = 256;
 constexpr int kNearMostCap = 65535;   // entries per particle (ncount's fields)
 constexpr int kNearShare = 8;   // age from which near lists are renewed with another system's
 constexpr float kListFar = 1.0e6f;
-// Neighbour cell of the cell pass, offsets within kMaxSpan: ox, oy, oz ascending.
-constexpr int kCodeSide = 2 * kMaxSpan + 1;
-__host__ __device__ inline int cell_code(int ox, int oy, int oz) {
-    return ((ox + kMaxSpan) * kCodeSide + (oy + kMaxSpan)) * kCodeSide + (oz + kMaxSpan);
+// Neighbour cell of the cell pass: its offset oz in the low 3 bits, oy in the
+// next ybits, ox in the rest (both signed), so that a code holds any x and y
+// offsets a grid can have.
+__host__ __device__ inline int cell_code(int ox, int oy, int oz, int ybits) {
+    return static_cast<int>(static_cast<unsigned>(ox) << (ybits + 3) |
+                            (static_cast<unsigned>(oy) & ((1u << ybits) - 1u)) << 3 | static_cast<unsigned>(oz + kMaxSpanZ));
 }
-constexpr int kOwnCell = (kMaxSpan * kCodeSide + kMaxSpan) * kCodeSide + kMaxSpan;   // cell_code(0, 0, 0)
+__host__ __device__ inline int code_x(int code, int ybits) { return code >> (ybits + 3); }
+__host__ __device__ inline int code_y(int code, int ybits) {
+    return static_cast<int>(static_cast<unsigned>(code) << (29 - ybits)) >> (32 - ybits);
+}
+__host__ __device__ inline int code_z(int code) { return (code & 7) - kMaxSpanZ; }
+constexpr int kOwnCell = kMaxSpanZ;    // cell_code(0, 0, 0, any)
 constexpr int kMaxBuildCells = 128;    // build stencil cells (at most 5^3)
 // Entry k of particle i: tiles of 64 particles of lcap * 256 bytes, inside a
 // tile batch by batch and a batch's particles in turn, so that a lane reads
@@ -186,7 +195,7 @@ struct NbLayout {
 template <typename real> struct KP {
     const SysDesc *sys;
     const int *cell_sys;
-    const int *stencil;   // cell codes of the pair pass, list codes of the list build
+    const int *stencil;   // cell codes of the cell pass, list codes of the list build
     const PotDesc<real> *pots;
     const int2 *slots;    // per system: descriptor slot -> (potential, next slot or 0)
     const real *coef;
@@ -220,6 +229,7 @@ template <typename real> struct KP {
     int coef_lds;     // 1 when every system's pair tables fit the LDS cache
     NbLayout nb;
     NbLayout nbs;     // cell pass: the staging area as one region, shared by a workgroup's waves
+    int part;         // cell pass: first stencil cell of the launch (kMaxSegCells at a time, the later launches add)
     // Neighbour lists (null and 0 without them).
     int list_mode;                    // (updates write buffer A in place)
     int light;                        // a light step: no binning, no build, skipped while a rebuild is due

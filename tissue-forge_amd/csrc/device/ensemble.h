@@ -86,6 +86,7 @@ struct DeviceEnsemble {
     int *d_list = nullptr, *d_lcount = nullptr, *d_cid0 = nullptr, *d_lflags = nullptr, *d_sflags = nullptr;
     int *d_ncount = nullptr;
     void *xb = nullptr, *x0 = nullptr, *xn = nullptr;
+    int max_stencil = 0;      // cells of the largest neighbour stencil
     int nb_cells = 4;         // cells of a pair-kernel workgroup
     int nonbond_resident = 0; // pair-kernel workgroups resident on the device at once
     LaunchShape shape;
@@ -210,7 +211,7 @@ template <typename real> int run_sync(DeviceEnsemble *E, const KP<real> &P, bool
 int run_count(DeviceEnsemble *E);
 template <typename real> int run_nonbond(DeviceEnsemble *E, const KP<real> &P);
 // Chooses the LDS layout and the resident grid of the pair kernel.
-template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_types, int max_coef, int max_stencil);
+template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_types, int max_coef);
 // update: 0 forces only, 1 forward-Euler update, 2..5 Runge-Kutta stage 1..4.
 template <typename real> int run_advance(DeviceEnsemble *E, const KP<real> &P, int update);
 // Neighbour lists: the build (a variant of the pair kernel over the wider

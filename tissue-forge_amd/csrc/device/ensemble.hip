@@ -89,6 +89,7 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy) {
     P.coef_lds = E->coef_lds_bytes > 0 ? 1 : 0;
     P.nb = E->nb;
     P.nbs = E->nbs;
+    P.part = 0;
     P.list_mode = E->list_mode ? 1 : 0;
     P.light = 0;
     P.lpp = E->lpp;
@@ -390,12 +391,15 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         d.share_above = d.np > kShareMean * d.ncells ? kShareAbove : INT_MAX;
         // Neighbour stencil: the cells whose closest point is inside the cutoff
         // (the task cull of tfSpace.cpp:949-954), as cell codes.
-        for (int k = 0; k < 3; k++)
-            if (e.geom.span[k] > kMaxSpan)
-                return set_error(TFG_E_RANGE, std::string("the cutoff spans more than 3 cells along ") + "xyz"[k]);
+        if (e.geom.span[2] > kMaxSpanZ)
+            return set_error(TFG_E_RANGE, "the cutoff spans more than 3 cells along z");
+        d.ybits = 2;
+        while (e.geom.span[1] >> (d.ybits - 1)) d.ybits++;
+        if (d.ybits > 26 || e.geom.span[0] >> (28 - d.ybits))   // (a stencil of hundreds of millions of cells)
+            return set_error(TFG_E_RANGE, "the cutoff spans too many cells along x and y");
         d.stencil_off = static_cast<int>(stencil.size());
         for (size_t k = 0; k < e.geom.stencil.size(); k += 3)
-            stencil.push_back(cell_code(e.geom.stencil[k], e.geom.stencil[k + 1], e.geom.stencil[k + 2]));
+            stencil.push_back(cell_code(e.geom.stencil[k], e.geom.stencil[k + 1], e.geom.stencil[k + 2], d.ybits));
         d.nstencil = static_cast<int>(stencil.size()) - d.stencil_off;
         max_stencil = std::max(max_stencil, d.nstencil);
         // Neighbour lists: build stencil for cutoff + skin (at most two cells
@@ -600,7 +604,8 @@ template <typename real> static int upload(DeviceEnsemble *E) {
     E->list_mode = list_ok && !E->no_alloc && !E->has_ext && np + 1 < (1 << kListSlotBits) &&
                    static_cast<size_t>(max_coef) * sizeof(real) <= 16384;
     E->lcap = E->list_mode ? lcap : 0;
-    int rc = nonbond_setup<real>(E, max_nt, max_coef, max_stencil);
+    E->max_stencil = max_stencil;
+    int rc = nonbond_setup<real>(E, max_nt, max_coef);
     if (rc != TFG_OK) return rc;
     if (E->list_mode && max_coef > 0 && E->coef_lds_bytes == 0) E->list_mode = false;
     // List pass blocks of 256 / lpp particles; lpp lanes per particle while

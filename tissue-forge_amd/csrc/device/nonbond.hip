@@ -170,7 +170,7 @@ NbLayout nb_layout(int max_nt, int coef_lds_count, int S, bool dpd, bool flux, b
         o->off_sp = b;
         if (flux) b += align16(chunk * S * static_cast<int>(sizeof(real)));
         o->off_seg = b;
-        b += align16(3 * max_stencil * 4);
+        b += align16(3 * std::min(max_stencil, kMaxSegCells) * 4);
         o->off_mark = b;
         b += align16(chunk / 32 * 4);
         // the slice reduction reuses the region: 64 lanes x (6 + S) values
@@ -389,11 +389,6 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
             const int per_pass = share ? group * kNbWaves : kWave;
             int loc[3];
             cell_loc(c - sd.cell_off, sd, loc);
-            // BUILD: the segment table of this cell's build stencil.  One lane
-            // per stencil cell loads its first slot and count (all in flight
-            // together); an inclusive scan gives each cell's end in the flat
-            // candidate order, so candidate t of the flat order is slot
-            // s_bbase[sg] + t of the cell sg with s_bend[sg - 1] <= t < s_bend[sg].
             // The first slot and the count of the stencil cell at offset o
             // (none beyond a non-periodic face: space_init's task list skips
             // it, tfSpace.cpp:913-944).
@@ -416,21 +411,23 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                     *cnt = P.start[cc + 1] - *first;
                 }
             };
-            // The cell pass: the non-empty stencil cells in order, each with
-            // its first candidate (the candidates of all cells in a row), the
-            // slot less candidate, and its code.  One lane per cell, so that
-            // the loads of all cells are in flight together.
             int *s_seg = reinterpret_cast<int *>(region + lay.off_seg);
             unsigned *s_mark = reinterpret_cast<unsigned *>(region + lay.off_mark);
-            int nseg = 0, total = 0, self_base = 0;   // self_base: candidate less slot in the own cell
-            (void)s_seg; (void)s_mark; (void)self_base;
+            (void)s_seg; (void)s_mark;
+            // The cell pass: the non-empty stencil cells of this launch's part
+            // in order, each with its first candidate (the candidates of all
+            // cells in a row), the slot less candidate, and its code.  One lane
+            // per cell, so that the loads of all cells are in flight together.
+            int nseg = 0, total = 0;
+            int self_base = -i0 - ni;   // candidate less slot in the own cell (none in this part)
+            (void)self_base;
             if constexpr (!BUILD) {
-                for (int h0 = 0; h0 < sd.nstencil; h0 += kWave) {
+                const int stop = min(sd.nstencil, P.part + kMaxSegCells);
+                for (int h0 = P.part; h0 < stop; h0 += kWave) {
                     int cnt = 0, first = 0, code = -1;
-                    if (h0 + lane < sd.nstencil) {
+                    if (h0 + lane < stop) {
                         code = P.stencil[sd.stencil_off + h0 + lane];
-                        const int o[3] = {code / (kCodeSide * kCodeSide) - kMaxSpan, code / kCodeSide % kCodeSide - kMaxSpan,
-                                          code % kCodeSide - kMaxSpan};
+                        const int o[3] = {code_x(code, sd.ybits), code_y(code, sd.ybits), code_z(code)};
                         stencil_cell(o, &first, &cnt);
                     }
                     int inc = cnt;
@@ -453,6 +450,11 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                 }
                 sync();
             }
+            // BUILD: the segment table of this cell's build stencil.  One lane
+            // per stencil cell loads its first slot and count (all in flight
+            // together); an inclusive scan gives each cell's end in the flat
+            // candidate order, so candidate t of the flat order is slot
+            // s_bbase[sg] + t of the cell sg with s_bend[sg - 1] <= t < s_bend[sg].
             int btotal = 0;
             if constexpr (BUILD) {
                 int carry = 0;
@@ -504,6 +506,17 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                 for (int k = 0; k < kMaxSpecies; k++) qacc[k] = real(0);
 
                 real fx = 0, fy = 0, fz = 0, nd = 0, ep = 0, vir = 0;
+                if (!BUILD && P.part > 0 && active && sl == 0) {   // on top of the earlier parts
+                    const v4 had = P.force[si];
+                    fx = had.x;
+                    fy = had.y;
+                    fz = had.z;
+                    nd = had.w;
+                    if (ENERGY) {
+                        ep = real(2.0 * P.e_nb[si]);
+                        vir = real(2.0 * P.e_vir[si]);
+                    }
+                }
                 int self_k = -1;   // staged index of the i particle itself in the current chunk
                 int lbase = 0;     // BUILD: list entries of this i particle so far
                 if (BUILD) s_self[lane] = -1;
@@ -1009,9 +1022,9 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                                 const int code = codev[u];
                                 v4 p = pv[u];
                                 if (EXT) s_rad[rel] = p.w;
-                                p.x = real(static_cast<double>(p.x) + (code / (kCodeSide * kCodeSide) - kMaxSpan) * sd.h[0]);
-                                p.y = real(static_cast<double>(p.y) + (code / kCodeSide % kCodeSide - kMaxSpan) * sd.h[1]);
-                                p.z = real(static_cast<double>(p.z) + (code % kCodeSide - kMaxSpan) * sd.h[2]);
+                                p.x = real(static_cast<double>(p.x) + code_x(code, sd.ybits) * sd.h[0]);
+                                p.y = real(static_cast<double>(p.y) + code_y(code, sd.ybits) * sd.h[1]);
+                                p.z = real(static_cast<double>(p.z) + code_z(code) * sd.h[2]);
                                 p.w = as_real_bits(type_column<v4>(mv[u].x & 0xffff), real(0));
                                 s_pos[rel] = p;
                                 if (kStageIds) s_id[rel] = mv[u].y;
@@ -1084,7 +1097,7 @@ __device__ __forceinline__ void nonbond_body(const KP<real> &P) {
                     fo.x = fx;
                     fo.y = fy;
                     fo.z = fz;
-                    fo.w = nd + real(sd.w_self);
+                    fo.w = nd + (P.part > 0 ? real(0) : real(sd.w_self));
                     P.force[si] = fo;
                     if (FLUX)
 #pragma unroll
@@ -1157,12 +1170,12 @@ static int variant_key(const DeviceEnsemble *E) {
     return (E->has_dpd ? 4 : 0) | (E->has_flux ? 2 : 0) | (E->has_ext ? 1 : 0);
 }
 
-template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_nt, int max_coef, int max_stencil) {
+template <typename real> int nonbond_setup(DeviceEnsemble *E, int max_nt, int max_coef) {
     const size_t cbytes = static_cast<size_t>(max_coef) * sizeof(real);
     E->coef_lds_bytes = (cbytes > 0 && cbytes <= static_cast<size_t>(kCoefLdsMax)) ? static_cast<int>(cbytes) : 0;
     const int max_chunk = 512;
     E->nb = nb_layout<real>(max_nt, E->coef_lds_bytes > 0 ? max_coef : 0, E->S, E->has_dpd, E->has_flux,
-                            E->has_ext, max_chunk, false, max_stencil, &E->nbs);
+                            E->has_ext, max_chunk, false, E->max_stencil, &E->nbs);
     // resident workgroups of the variant that runs every step (no energies)
     const void *fn = pick_nonbond<real>(variant_key(E), E->coef_lds_bytes > 0, false);
     int per_cu = 0;
@@ -1185,10 +1198,13 @@ int nonbond_waves() { return kNbWaves; }
 
 template <typename real> int run_nonbond(DeviceEnsemble *E, const KP<real> &P) {
     const void *fn = pick_nonbond<real>(variant_key(E), P.coef_lds != 0, P.energy != 0);
-    void *args[] = {const_cast<KP<real> *>(&P)};
-    const hipError_t e =
-        hipLaunchKernel(fn, dim3(E->nonbond_grid()), dim3(kNbThreads), args, E->nb.total, E->stream);
-    if (e != hipSuccess) return set_error(TFG_E_DEVICE, std::string("nonbond: ") + hipGetErrorString(e));
+    KP<real> Q = P;
+    void *args[] = {&Q};
+    for (Q.part = 0; Q.part < E->max_stencil; Q.part += kMaxSegCells) {
+        const hipError_t e =
+            hipLaunchKernel(fn, dim3(E->nonbond_grid()), dim3(kNbThreads), args, E->nb.total, E->stream);
+        if (e != hipSuccess) return set_error(TFG_E_DEVICE, std::string("nonbond: ") + hipGetErrorString(e));
+    }
     return launch_error("nonbond");
 }
 
@@ -1747,7 +1763,7 @@ template int run_list_build<float>(DeviceEnsemble *, const KP<float> &);
 template int run_list_build<double>(DeviceEnsemble *, const KP<double> &);
 template int run_nonbond<float>(DeviceEnsemble *, const KP<float> &);
 template int run_nonbond<double>(DeviceEnsemble *, const KP<double> &);
-template int nonbond_setup<float>(DeviceEnsemble *, int, int, int);
-template int nonbond_setup<double>(DeviceEnsemble *, int, int, int);
+template int nonbond_setup<float>(DeviceEnsemble *, int, int);
+template int nonbond_setup<double>(DeviceEnsemble *, int, int);
 
 }  // namespace tfg
