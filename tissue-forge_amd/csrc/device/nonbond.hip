@@ -156,7 +156,7 @@ NbLayout nb_layout(int max_nt, int coef_lds_count, int S, bool dpd, bool flux, b
     L.coef_half = coef_lds_count / 2 * static_cast<int>(sizeof(real));   // a whole number of 4-vectors
     L.off_waves = L.off_coef + align16(coef_lds_count * static_cast<int>(sizeof(real)));
     if (build) L.off_waves += align16(125 * static_cast<int>(sizeof(v4)));   // shifts of the 125 build-cell offsets
-    auto region = [&](int chunk, NbLayout *o) {
+    auto region = [&](int chunk, int cells, NbLayout *o) {   // cells: the segment table's
         int b = align16((chunk + kPad) * static_cast<int>(sizeof(v4)));
         o->off_id = b;
         if (ids) b += align16(chunk * 4);
@@ -170,22 +170,25 @@ NbLayout nb_layout(int max_nt, int coef_lds_count, int S, bool dpd, bool flux, b
         o->off_sp = b;
         if (flux) b += align16(chunk * S * static_cast<int>(sizeof(real)));
         o->off_seg = b;
-        b += align16(3 * std::min(max_stencil, kMaxSegCells) * 4);
+        b += align16(3 * cells * 4);
         o->off_mark = b;
         b += align16(chunk / 32 * 4);
         // the slice reduction reuses the region: 64 lanes x (6 + S) values
         return std::max(b, kWave * (6 + S) * static_cast<int>(sizeof(real)));
     };
+    // The chunk is chosen beside the smallest stencil's table: it divides the
+    // candidates into sums, so it must not follow from the other systems of the
+    // ensemble.  A larger table comes on top of the budget.
+    const int cells = std::min(max_stencil, kMaxSegCells);
     int chunk = max_chunk;
-    while (chunk > 64 && kNbWaves * region(chunk, &L) > kWaveLdsBudget) chunk /= 2;
+    while (chunk > 64 && kNbWaves * region(chunk, std::min(cells, 27), &L) > kWaveLdsBudget) chunk /= 2;
     L.chunk = chunk;
-    L.region = region(chunk, &L);
+    L.region = region(chunk, cells, &L);
     L.total = L.off_waves + kNbWaves * L.region;
-    if (shared) {   // the waves' regions as one, of as many entries as they hold
+    if (shared) {   // the waves' regions as one, of as many entries
         *shared = L;
-        int most = kNbWaves * chunk;
-        while (region(most, shared) > kNbWaves * L.region) most -= kWave;
-        shared->chunk = most;
+        shared->chunk = kNbWaves * chunk;
+        region(shared->chunk, cells, shared);
     }
     return L;
 }
