@@ -56,6 +56,10 @@ struct LaunchShape {
     int stream_blocks = 0;
 };
 
+// A member's last read: none since its host record, of the state it has now,
+// of an earlier state that is kept.
+constexpr char kReadNone = 0, kReadCurrent = 1, kReadKept = 2;
+
 struct DeviceEnsemble {
     int precision = PREC_MIXED;
     int device = 0;
@@ -149,13 +153,12 @@ struct DeviceEnsemble {
         hipEvent_t done = nullptr;
     };
     ReadSlot read_slot[8];
-    // keep_reads: the state of each member at its last read, by id on the
-    // device (kept, with its energies), for host engines that leave the
-    // ensemble without a download.
+    // keep_reads: what was last read of a member is what its host engine holds
+    // when it leaves the ensemble without a download.  kept: that state by id
+    // on the device, for the members whose state has changed since (kept_sys).
     bool keep_reads = false;
     ReadRows kept;
-    double *kept_energy = nullptr;
-    std::vector<char> kept_sys;
+    std::vector<char> kept_sys;   // kReadNone ..
 
     ~DeviceEnsemble() {
         if (status) (void)hipHostFree(status);
@@ -198,8 +201,10 @@ template <typename real> KP<real> make_params(DeviceEnsemble *E, int energy);
 int ensemble_force_arena(Engine *e, int precision, void *arena, size_t cap, double *f, Energies *en);
 
 // Readback (readback.hip): system s from the device into its host engine's
-// particles, and for keep_reads its state kept on the device and put back.
+// particles; for keep_reads the members read are kept before their state
+// changes, and put back at the end.
 int read_into_engine(DeviceEnsemble *E, int s);
+int keep_reads(DeviceEnsemble *E);
 int restore_kept(DeviceEnsemble *E);
 
 // Binning: scan of the cell counts, placement, per-cell order and move of

@@ -1056,7 +1056,9 @@ int ensemble_step(DeviceEnsemble *E, int nsteps, bool use_graph) {
     if (nsteps < 0) return set_error(TFG_E_INVALIDARG, "negative step count");
     if (nsteps == 0) return TFG_OK;
     TFG_HIP(hipSetDevice(E->device));
-    const int rc = E->precision == PREC_MIXED ? step_t<float>(E, nsteps, use_graph) : step_t<double>(E, nsteps, use_graph);
+    int rc = keep_reads(E);
+    if (rc != TFG_OK) return rc;
+    rc = E->precision == PREC_MIXED ? step_t<float>(E, nsteps, use_graph) : step_t<double>(E, nsteps, use_graph);
     if (rc == TFG_E_DEVICE) return rc;
     // also after a failed step: the host time counts the steps begun
     const std::string msg = rc != TFG_OK ? std::string(last_error()) : std::string();
@@ -1140,6 +1142,8 @@ int ensemble_force_arena(Engine *e, int precision, void *arena, size_t cap, doub
 
 int ensemble_force(DeviceEnsemble *E) {
     TFG_HIP(hipSetDevice(E->device));
+    const int rc = keep_reads(E);
+    if (rc != TFG_OK) return rc;
     return E->precision == PREC_MIXED ? force_t<float>(E) : force_t<double>(E);
 }
 
@@ -1175,6 +1179,8 @@ int ensemble_species_totals(DeviceEnsemble *E, int s, double *out, int cap) {
 int ensemble_autotune(DeviceEnsemble *E, int reps, int *blocks_out, int *stream_blocks_out) {
     if (reps < 1) reps = 1;
     TFG_HIP(hipSetDevice(E->device));
+    const int kept = keep_reads(E);
+    if (kept != TFG_OK) return kept;
     auto run = [&](int which) -> double {
         double best = 1e30;
         for (int r = 0; r < reps; r++) {

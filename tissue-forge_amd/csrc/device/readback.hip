@@ -256,8 +256,7 @@ static void record_rows(Engine &e, const ReadRows &r, int first, int n) {
     }
 }
 
-int read_into_engine(DeviceEnsemble *E, int s) {
-    const std::lock_guard<std::mutex> hold(E->read_lock);
+static int read_into_engine_locked(DeviceEnsemble *E, int s) {
     Engine &e = *E->engines[s];
     double some = 0;
     int some_i = 0;
@@ -267,8 +266,13 @@ int read_into_engine(DeviceEnsemble *E, int s) {
     want.ns = e.nspecies;
     if (e.nspecies > 0) want.sp = want.q = &some;
     const int rc = read_system(E, s, want, [&](const ReadRows &r, int first, int n) { record_rows(e, r, first, n); });
-    if (rc == TFG_OK && !E->kept_sys.empty()) E->kept_sys[s] = 0;   // the host record is newer
+    if (rc == TFG_OK && E->keep_reads) E->kept_sys[s] = kReadNone;   // the host record is newer
     return rc;
+}
+
+int read_into_engine(DeviceEnsemble *E, int s) {
+    const std::lock_guard<std::mutex> hold(E->read_lock);
+    return read_into_engine_locked(E, s);
 }
 
 // The member's rows inside the kept arrays (id order over the ensemble).
@@ -286,40 +290,66 @@ static ReadRows kept_rows(const DeviceEnsemble *E, int s) {
     return r;
 }
 
-void ensemble_keep_reads(DeviceEnsemble *E) { E->keep_reads = true; }
+void ensemble_keep_reads(DeviceEnsemble *E) {
+    E->keep_reads = true;
+    E->kept_sys.assign(E->nsys, kReadNone);
+}
 
-static int keep_read(DeviceEnsemble *E, int s) {
-    const OnDevice on(E->device);
-    int rc;
-    if (E->kept_sys.empty()) {
-        const size_t n = static_cast<size_t>(E->np);
-        ReadRows &k = E->kept;
-        if ((rc = E->buf.alloc(&k.x, 3 * n)) != TFG_OK || (rc = E->buf.alloc(&k.v, 3 * n)) != TFG_OK ||
-            (rc = E->buf.alloc(&k.f, 4 * n)) != TFG_OK || (rc = E->buf.alloc(&k.cid, n)) != TFG_OK ||
-            (rc = E->buf.alloc(&k.flags, n)) != TFG_OK || (rc = E->buf.alloc(&k.sp, n * E->S)) != TFG_OK ||
-            (rc = E->buf.alloc(&k.q, n * E->S)) != TFG_OK ||
-            (rc = E->buf.alloc(&E->kept_energy, static_cast<size_t>(5) * E->nsys)) != TFG_OK)
-            return rc;
-        E->kept_sys.assign(E->nsys, 0);
+// The kept arrays, one block, on first use; false without device memory for it.
+static bool kept_alloc(DeviceEnsemble *E) {
+    if (E->kept.x) return true;
+    const size_t n = static_cast<size_t>(E->np);
+    double *p = nullptr;
+    if (E->buf.alloc(&p, n * (11 + 2 * E->S)) != TFG_OK) {
+        (void)hipGetLastError();   // the caller goes on without it
+        return false;
     }
-    if ((rc = launch_read(E, s, 0, E->sys[s].np, kept_rows(E, s), E->stream)) != TFG_OK) return rc;
-    TFG_HIP(hipMemcpyAsync(E->kept_energy + 5 * s, E->d_energy + 5 * s, 5 * sizeof(double), hipMemcpyDeviceToDevice,
-                           E->stream));
-    E->kept_sys[s] = 1;
+    ReadRows &k = E->kept;
+    k.x = p;
+    k.v = k.x + 3 * n;
+    k.f = k.v + 3 * n;
+    k.sp = k.f + 4 * n;
+    k.q = k.sp + n * E->S;
+    k.cid = reinterpret_cast<int *>(k.q + n * E->S);
+    k.flags = k.cid + n;
+    return true;
+}
+
+// A read copies nothing for later: the state of the members read is kept here,
+// by the next call that changes it (sweeps read every member between two
+// steps, and a gather behind each read delayed the next one).  Without device
+// memory the host engines take it now.
+int keep_reads(DeviceEnsemble *E) {
+    if (!E->keep_reads) return TFG_OK;
+    const std::lock_guard<std::mutex> hold(E->read_lock);
+    for (int s = 0; s < E->nsys; s++) {
+        if (E->kept_sys[s] != kReadCurrent) continue;
+        int rc;
+        if (kept_alloc(E)) {
+            rc = launch_read(E, s, 0, E->sys[s].np, kept_rows(E, s), E->stream);
+            if (rc == TFG_OK) E->kept_sys[s] = kReadKept;
+        } else {
+            rc = read_into_engine_locked(E, s);
+        }
+        if (rc != TFG_OK) return rc;
+    }
     return TFG_OK;
 }
 
 int restore_kept(DeviceEnsemble *E) {
     const std::lock_guard<std::mutex> hold(E->read_lock);
     for (int s = 0; s < static_cast<int>(E->kept_sys.size()); s++) {
-        if (!E->kept_sys[s]) continue;
+        if (E->kept_sys[s] == kReadCurrent) {
+            const int rc = read_into_engine_locked(E, s);
+            if (rc != TFG_OK) return rc;
+        }
+        if (E->kept_sys[s] != kReadKept) continue;
         const OnDevice on(E->device);
         Engine &e = *E->engines[s];
         const size_t n = static_cast<size_t>(E->sys[s].np);
         const ReadRows d = kept_rows(E, s);
         std::vector<double> x(3 * n), v(3 * n), f(4 * n), sp(n * d.ns), q(n * d.ns);
         std::vector<int> cid(n), flags(n);
-        double en[5];
         ReadRows h;
         h.x = x.data(), h.v = v.data(), h.f = f.data(), h.sp = sp.data(), h.q = q.data();
         h.cid = cid.data(), h.flags = flags.data();
@@ -334,9 +364,7 @@ int restore_kept(DeviceEnsemble *E) {
             TFG_HIP(hipMemcpy(h.sp, d.sp, n * d.ns * sizeof(double), hipMemcpyDeviceToHost));
             TFG_HIP(hipMemcpy(h.q, d.q, n * d.ns * sizeof(double), hipMemcpyDeviceToHost));
         }
-        TFG_HIP(hipMemcpy(en, E->kept_energy + 5 * s, sizeof(en), hipMemcpyDeviceToHost));
         record_rows(e, h, 0, static_cast<int>(n));
-        e.energies = energies_of(en);
     }
     return TFG_OK;
 }
@@ -345,7 +373,11 @@ int ensemble_read(DeviceEnsemble *E, int s, const ReadRows &out) {
     if (s < 0 || s >= E->nsys) return set_error(TFG_E_RANGE, "system index out of range");
     const std::lock_guard<std::mutex> hold(E->read_lock);
     const int rc = read_system(E, s, out, [&](const ReadRows &rows, int first, int n) { copy_rows(rows, out, first, n); });
-    return rc == TFG_OK && E->keep_reads ? keep_read(E, s) : rc;
+    if (rc == TFG_OK && E->keep_reads) {
+        E->kept_sys[s] = kReadCurrent;
+        E->engines[s]->energies = energies_of(E->status_sums() + 5 * s);
+    }
+    return rc;
 }
 
 }  // namespace tfg
