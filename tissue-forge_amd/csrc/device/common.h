@@ -24,15 +24,25 @@ constexpr int kWave = 64;
 constexpr int kMaxTypes = 8;          // type pairs cached in LDS by the pair kernel
 constexpr int kMaxSpecies = 8;        // TF_SIMD_SIZE
 constexpr int kMaxFluxEntries = 64;   // flux entries per system
-// Cell pass of crowded systems (more than kShareMean particles per cell on
+// Cell pass of crowded systems (more than share_mean particles per cell on
 // average at the upload): a cell of more than kShareAbove particles is one
 // workgroup's.  One wave per cell leaves such systems with few waves, each
-// long: 8,000 particles 199 us a step, shared 75; 30,000 190, 77; 200,000
-// 341, 209.  At 16 per cell sharing leaves a lane too few candidates
-// (1,000,000 particles 0.63 ms, shared 0.93), so those keep the wave.
+// long; shared, a lane of a sparser cell has too few candidates, and the more
+// cells there are the less it matters that a wave is long.  Force passes in
+// microseconds, a wave per cell and shared, Morse FP32 / DPD with a flux FP64:
+//   cells   12 per cell        14                 17                 19.5
+//   64      88, 76 / 160, 114  96, 79 / 189, 128  139, 84 / 310, 141 150, 81 / 344, 135
+//   1,000   100, 91 / 189, 175 105, 99 / 208, 198 146, 97 / 323, 207 160, 103 / 373, 226
+//   1,728   102, 109 / 198, 229 106, 109 / 226, 250 149, 117 / 357, 268 163, 122 / 394, 292
+//   4,096   113, 143 / 276, 387 120, 151 / 350, 432 159, 156 / 483, 456 197, 162 / 565, 508
+// and with radii in FP64 17 per cell 181, 168 (1,000 cells), 202, 221 (1,728),
+// 400, 386 (4,096); 8,000 cells of DPD with a flux in FP64 at 17 694, 770, at
+// 20.5 1,005, 886; 64,000 Morse cells at 15.6 0.63 ms, 0.93.
 // The rule looks at the system alone, so that its results do not depend on
 // the ensemble it is in.
-constexpr double kShareMean = 20.0;
+__host__ inline double share_mean(int ncells) {
+    return ncells <= 1024 ? 14.0 : ncells <= 2048 ? 16.0 : ncells <= 4096 ? 18.0 : 20.0;
+}
 constexpr int kShareAbove = 12;
 constexpr int kMaxSpanZ = 3;          // cells of cutoff along z per direction
 constexpr int kMaxSegCells = 343;     // stencil cells of the cell pass's segment table; larger stencils take several launches

@@ -386,9 +386,9 @@ template <typename real> static int upload(DeviceEnsemble *E) {
         d.p_off = np;
         d.np = static_cast<int>(e.parts.size());
         d.ntypes = nt;
-        // Crowded systems (more than kShareMean particles per cell): the whole
-        // workgroup takes each cell of more than kShareAbove.
-        d.share_above = d.np > kShareMean * d.ncells ? kShareAbove : INT_MAX;
+        // Crowded systems: the whole workgroup takes each cell of more than
+        // kShareAbove particles.
+        d.share_above = d.np > share_mean(d.ncells) * d.ncells ? kShareAbove : INT_MAX;
         // Neighbour stencil: the cells whose closest point is inside the cutoff
         // (the task cull of tfSpace.cpp:949-954), as cell codes.
         if (e.geom.span[2] > kMaxSpanZ)
