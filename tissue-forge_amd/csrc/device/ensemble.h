@@ -142,6 +142,8 @@ struct DeviceEnsemble {
     Status *status = nullptr;
     double *status_sums() const { return reinterpret_cast<double *>(status + 1); }
     int light_run = 4;   // light steps between two full ones
+    bool full_only = false;   // no light steps: almost every step waits (of the last sample, counted here)
+    int sample_steps = 0, sample_waits = 0;
 
     // Readback: a pinned buffer and an event per reading thread.  read_lock is
     // held over a read: host threads may read several members, or one engine

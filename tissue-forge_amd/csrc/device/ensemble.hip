@@ -907,12 +907,17 @@ template <typename real> static int step_graph(DeviceEnsemble *E) {
 // come out the same, whichever slot runs them.  A run of light steps between
 // full ones costs the chain once per run, and each rebuild wastes half a run
 // of launches that do nothing: with ~17 us and ~4 us that is least at
-// sqrt(8 x the steps from one wait to the next).  Where less than 1.5 steps lie
-// between two waits (thin skins, ensembles of hundreds of members) light slots
-// only get in the way and there are none: 20,000 DPD particles with a skin of
-// 0.02 78 us a step with runs of two, 67 without, 256 replicas 361, 349.  Every
-// slot runs one step at most, so the call sends as many slots as steps are left,
-// looks at the counter, and sends the rest.
+// sqrt(8 x the steps from one wait to the next).  Every slot runs one step at
+// most, so the call sends as many slots as steps are left, looks at the counter,
+// and sends the rest.
+//
+// Where less than 1.5 steps lie between two waits (thin skins, ensembles of
+// hundreds of members) light slots only get in the way and there are none:
+// 20,000 DPD particles with a skin of 0.02 78 us a step with runs of two, 67
+// without, 256 replicas 361, 349.  That is decided over kWaitSample steps (the
+// first steps of a system all wait), and looked at again after kFullSlots, since
+// full steps alone cost 8,000 settled particles 45 us a step in place of 32.
+constexpr int kWaitSample = 16, kFullSlots = 64;
 template <typename real> static int list_steps(DeviceEnsemble *E, int nsteps) {
     int rc;
     KP<real> L = make_params<real>(E, 0);
@@ -921,8 +926,9 @@ template <typename real> static int list_steps(DeviceEnsemble *E, int nsteps) {
     for (int left = nsteps; left > 0;) {
         const DeviceEnsemble::Status before = *E->status;
         bool full = before.due != 0;
-        for (int k = 0, run = 0; k < left - 1; k++) {
-            if (full || run >= E->light_run) {
+        const int slots = E->full_only ? std::min(left, kFullSlots) : left;
+        for (int k = 0, run = 0; k < slots - 1; k++) {
+            if (full || E->full_only || run >= E->light_run) {
                 if ((rc = step_graph<real>(E)) != TFG_OK) return rc;
                 TFG_HIP(hipGraphLaunch(E->graph, E->stream));
                 full = false;
@@ -938,11 +944,15 @@ template <typename real> static int list_steps(DeviceEnsemble *E, int nsteps) {
         const int done = static_cast<int>(now.step - before.step), served = now.served - before.served;
         if (done < 1 || done > left) return set_error(TFG_E_DEVICE, "list steps: the step counter is off");
         left -= done;
-        if (served > 0) {
-            const double apart = static_cast<double>(done) / served;
-            E->light_run = apart < 1.5 ? 0 : std::min(32, static_cast<int>(std::sqrt(8.0 * apart)));
-        } else if (done > E->light_run) {
-            E->light_run = std::min(32, std::max(1, 2 * E->light_run));
+        if (served > 0)
+            E->light_run = std::max(1, std::min(32, static_cast<int>(std::sqrt(8.0 * done / served))));
+        else if (done > E->light_run)
+            E->light_run = std::min(32, 2 * E->light_run);
+        E->sample_steps += done;
+        E->sample_waits += served;
+        if (E->sample_steps >= kWaitSample) {
+            E->full_only = E->sample_steps < 1.5 * E->sample_waits;
+            E->sample_steps = E->sample_waits = 0;
         }
     }
     return TFG_OK;
