@@ -335,7 +335,7 @@ __global__ __launch_bounds__(64) void k_order(KP<real> P, const int *gate) {
 
 // Buffer B brought up to date from A after in-place updates (lflags[3]):
 // before a rebuilding step's binning (all reads of B follow), or always
-// (force, a force pass or a download).  Nothing to do while B is current.
+// (force: a force pass).  Nothing to do while B is current.
 template <typename real>
 __global__ void k_sync(KP<real> P, int force) {
     if (P.lflags[3] == 0) return;

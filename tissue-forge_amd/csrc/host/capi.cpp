@@ -99,7 +99,7 @@ int tfg_engine_destroy(tfg_engine *h) {
         // released through its ensemble first.
         if (ensemble_size(h->e.device) != 1)
             return set_error(TFG_E_STATE, "engine belongs to an ensemble; destroy the ensemble first");
-        if (ensemble_destroy(h->e.device, false) != TFG_OK) return TFG_E_DEVICE;
+        TFG_GUARD(if (ensemble_destroy(h->e.device, false) != TFG_OK) return TFG_E_DEVICE);
     }
     delete h;
     return TFG_OK;
@@ -815,9 +815,10 @@ int tfg_ensemble_step(tfg_ensemble *ens, int nsteps, int use_graph) {
 
 int tfg_ensemble_destroy(tfg_ensemble *ens, int download) {
     if (!ens) return TFG_OK;
-    DeviceEnsemble *dev = ens->dev;
+    int rc = TFG_OK;
+    TFG_GUARD(rc = ensemble_destroy(ens->dev, download != 0));   // (out of host memory: still there, to try again)
     delete ens;
-    TFG_GUARD(return ensemble_destroy(dev, download != 0));
+    return rc;
 }
 
 double tfg_ensemble_last_ms(const tfg_ensemble *ens) {
