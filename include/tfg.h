@@ -345,7 +345,8 @@ int tfg_nonbond_eval(tfg_engine *e);
  * TFG_E_INVALIDARG for an engine with no particles. */
 int tfg_nonbond_eval_noalloc(tfg_engine *e, int precision, double *f, double energies[6]);
 
-/* ---- readback (synchronous). ---- */
+/* ---- readback (synchronous).  Reads may be made from several host threads at
+ *      once, also of several members of one ensemble. ---- */
 /* out[0..5] = epot, epot_nonbond, epot_bond, epot_angle, ekin, virial of the
  * last evaluated step (space epot fields, source/mdcore/include/tfSpace.h:207;
  * engine_kinetic_energy, source/mdcore/src/tfEngine.cpp:1893-1927). */
