@@ -76,3 +76,34 @@ def test_without_device_memory(gpu, tf, W):
     ens.step(1)
     ens.close(download=False)
     assert equal(engines[1].particles(), p)
+
+
+def test_species_of_different_members(gpu, tf, W):
+    """Members of 0, 1 and 3 species, one of them not read before the change."""
+    def scene(n, S):
+        sc = W.dpd_droplets(n=n, density=3.0, seed=n, radius=2.0)
+        if S == 0:
+            return dict(sc, nspecies=0, fluxes=[], species=None)
+        return dict(sc, nspecies=S, species=np.random.default_rng(n).uniform(size=(n, S)))
+    shapes = [(700, 1), (1500, 3), (600, 0), (900, 3)]
+    engines = [W.build_engine(scene(n, S))[0] for n, S in shapes]
+    host = W.build_engine(scene(*shapes[3]))[0].particles()
+    ens = tf.Ensemble(engines, tf.PREC_FP64)
+    ens.step(2)
+    read = [e.particles() for e in engines[:3]]
+    ens.step(2)
+    ens.close(download=False)
+    for e, want in zip(engines, read + [host]):
+        assert equal(e.particles(), want)
+
+
+def test_many_members(gpu, tf, W):
+    """More members than one launch keeps (256), a part of them read."""
+    engines = members(W, [200 + k % 7 for k in range(300)])
+    ens = tf.Ensemble(engines, tf.PREC_MIXED)
+    ens.step(1)
+    read = {k: engines[k].particles() for k in (0, 31, 32, 130, 255, 256, 299)}
+    ens.step(1)
+    ens.close(download=False)
+    for k, want in read.items():
+        assert equal(engines[k].particles(), want), k

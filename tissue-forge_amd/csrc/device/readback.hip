@@ -46,19 +46,32 @@ __device__ inline void put_rows(T *out, int first, int n, const T0 (&v)[W], T *l
     for (int t = threadIdx.x; t < n * W; t += kReadBlock) out[static_cast<size_t>(first) * W + t] = lds[t];
 }
 
-// Ids [id0, id0 + n) of system s into the rows of o (null fields skipped).
-// Positions follow the host's arithmetic: stored + frame offset, then
-// (origin + loc h) + x, each rounded once.
-template <typename real> __global__ __launch_bounds__(kReadBlock) void k_read(KP<real> P, int s, int id0, int n, ReadRows o) {
+// The rows from particle p on (kept.ns species per row).
+__host__ __device__ inline ReadRows kept_at(const ReadRows &kept, size_t p) {
+    ReadRows r = kept;
+    r.x += 3 * p;
+    r.v += 3 * p;
+    r.f += 4 * p;
+    r.cid += p;
+    r.flags += p;
+    if (r.ns > 0) {
+        r.sp += r.ns * p;
+        r.q += r.ns * p;
+    }
+    return r;
+}
+
+// Ids [id0, id0 + n) of a system into the rows of o (null fields skipped), by
+// the block of ids b0 / kReadBlock.  Positions follow the host's arithmetic:
+// stored + frame offset, then (origin + loc h) + x, each rounded once.
+template <typename real>
+__device__ inline void read_block(const KP<real> &P, const SysDesc &sd, int id0, int n, int b0, const ReadRows &o, double *lds) {
 #pragma clang fp contract(off)
-    __shared__ double lds[kReadBlock * 4];
-    const SysDesc &sd = P.sys[s];
     const bool from_a = P.list_mode && P.lflags[3] != 0;   // in-place updates leave B behind A
     const typename V<real>::v4 *pos = from_a ? P.A.pos : P.B.pos;
     const typename V<real>::v4 *vel = from_a ? P.A.vel : P.B.vel;
     const int4 *meta = from_a ? P.A.meta : P.B.meta;
     const real *sp = from_a ? P.A.sp : P.B.sp, *q = from_a ? P.A.q : P.B.q;
-    const int b0 = blockIdx.x * kReadBlock;
     const int nb = min(kReadBlock, n - b0);
     const bool valid = static_cast<int>(threadIdx.x) < nb;
     const int slot = P.slot_of[sd.p_off + id0 + b0 + (valid ? static_cast<int>(threadIdx.x) : 0)];
@@ -99,6 +112,28 @@ template <typename real> __global__ __launch_bounds__(kReadBlock) void k_read(KP
     }
 }
 
+template <typename real> __global__ __launch_bounds__(kReadBlock) void k_read(KP<real> P, int s, int id0, int n, ReadRows o) {
+    __shared__ double lds[kReadBlock * 4];
+    read_block<real>(P, P.sys[s], id0, n, blockIdx.x * kReadBlock, o, lds);
+}
+
+// The marked ones of kKeepGroup members into the kept arrays (id order over the
+// ensemble, P.S species per row), in one launch: a launch per member cost the
+// step after the reads of 49 members 0.15 ms.
+constexpr int kKeepGroup = 256;
+struct Marks {
+    unsigned bits[kKeepGroup / 32];
+};
+template <typename real> __global__ __launch_bounds__(kReadBlock) void k_keep(KP<real> P, int first, Marks marks, ReadRows kept) {
+    __shared__ double lds[kReadBlock * 4];
+    const int g = blockIdx.y;
+    if ((marks.bits[g >> 5] >> (g & 31) & 1u) == 0) return;
+    const SysDesc &sd = P.sys[first + g];
+    const int b0 = blockIdx.x * kReadBlock;
+    if (b0 >= sd.np) return;
+    read_block<real>(P, sd, 0, sd.np, b0, kept_at(kept, sd.p_off), lds);
+}
+
 int launch_read(DeviceEnsemble *E, int s, int id0, int n, const ReadRows &o, hipStream_t stream) {
     const dim3 g((n + kReadBlock - 1) / kReadBlock), b(kReadBlock);
     if (E->precision == PREC_MIXED)
@@ -106,6 +141,15 @@ int launch_read(DeviceEnsemble *E, int s, int id0, int n, const ReadRows &o, hip
     else
         hipLaunchKernelGGL(k_read<double>, g, b, 0, stream, make_params<double>(E, 0), s, id0, n, o);
     return launch_error("readback");
+}
+
+int launch_keep(DeviceEnsemble *E, int first, int count, int most, const Marks &m) {
+    const dim3 g((most + kReadBlock - 1) / kReadBlock, count), b(kReadBlock);
+    if (E->precision == PREC_MIXED)
+        hipLaunchKernelGGL(k_keep<float>, g, b, 0, E->stream, make_params<float>(E, 0), first, m, E->kept);
+    else
+        hipLaunchKernelGGL(k_keep<double>, g, b, 0, E->stream, make_params<double>(E, 0), first, m, E->kept);
+    return launch_error("kept reads");
 }
 
 // The wanted fields of o (non-null) laid one after the other in a buffer for
@@ -275,21 +319,6 @@ int read_into_engine(DeviceEnsemble *E, int s) {
     return read_into_engine_locked(E, s);
 }
 
-// The member's rows inside the kept arrays (id order over the ensemble).
-static ReadRows kept_rows(const DeviceEnsemble *E, int s) {
-    const size_t p = static_cast<size_t>(E->sys[s].p_off);
-    ReadRows r = E->kept;
-    r.ns = E->engines[s]->nspecies;
-    r.x += 3 * p;
-    r.v += 3 * p;
-    r.f += 4 * p;
-    r.cid += p;
-    r.flags += p;
-    r.sp = r.ns > 0 ? r.sp + p * E->S : nullptr;
-    r.q = r.ns > 0 ? r.q + p * E->S : nullptr;
-    return r;
-}
-
 void ensemble_keep_reads(DeviceEnsemble *E) {
     E->keep_reads = true;
     E->kept_sys.assign(E->nsys, kReadNone);
@@ -312,6 +341,7 @@ static bool kept_alloc(DeviceEnsemble *E) {
     k.q = k.sp + n * E->S;
     k.cid = reinterpret_cast<int *>(k.q + n * E->S);
     k.flags = k.cid + n;
+    k.ns = E->S;
     return true;
 }
 
@@ -322,16 +352,24 @@ static bool kept_alloc(DeviceEnsemble *E) {
 int keep_reads(DeviceEnsemble *E) {
     if (!E->keep_reads) return TFG_OK;
     const std::lock_guard<std::mutex> hold(E->read_lock);
-    for (int s = 0; s < E->nsys; s++) {
-        if (E->kept_sys[s] != kReadCurrent) continue;
-        int rc;
-        if (kept_alloc(E)) {
-            rc = launch_read(E, s, 0, E->sys[s].np, kept_rows(E, s), E->stream);
-            if (rc == TFG_OK) E->kept_sys[s] = kReadKept;
-        } else {
-            rc = read_into_engine_locked(E, s);
+    if (std::find(E->kept_sys.begin(), E->kept_sys.end(), kReadCurrent) == E->kept_sys.end()) return TFG_OK;
+    const bool device = kept_alloc(E);
+    for (int first = 0; first < E->nsys; first += kKeepGroup) {
+        const int count = std::min(kKeepGroup, E->nsys - first);
+        Marks marks{};
+        int most = 0, rc;
+        for (int g = 0; g < count; g++) {
+            char &state = E->kept_sys[first + g];
+            if (state != kReadCurrent) continue;
+            if (!device) {
+                if ((rc = read_into_engine_locked(E, first + g)) != TFG_OK) return rc;
+                continue;
+            }
+            marks.bits[g >> 5] |= 1u << (g & 31);
+            most = std::max(most, E->sys[first + g].np);
+            state = kReadKept;
         }
-        if (rc != TFG_OK) return rc;
+        if (most > 0 && (rc = launch_keep(E, first, count, most, marks)) != TFG_OK) return rc;
     }
     return TFG_OK;
 }
@@ -347,23 +385,29 @@ int restore_kept(DeviceEnsemble *E) {
         const OnDevice on(E->device);
         Engine &e = *E->engines[s];
         const size_t n = static_cast<size_t>(E->sys[s].np);
-        const ReadRows d = kept_rows(E, s);
-        std::vector<double> x(3 * n), v(3 * n), f(4 * n), sp(n * d.ns), q(n * d.ns);
+        const ReadRows d = kept_at(E->kept, E->sys[s].p_off);
+        const size_t S = d.ns;
+        std::vector<double> x(3 * n), v(3 * n), f(4 * n), sp(n * S), q(n * S);
         std::vector<int> cid(n), flags(n);
         ReadRows h;
         h.x = x.data(), h.v = v.data(), h.f = f.data(), h.sp = sp.data(), h.q = q.data();
         h.cid = cid.data(), h.flags = flags.data();
-        h.ns = d.ns;
+        h.ns = e.nspecies;
         TFG_HIP(hipStreamSynchronize(E->stream));
         TFG_HIP(hipMemcpy(h.x, d.x, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
         TFG_HIP(hipMemcpy(h.v, d.v, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
         TFG_HIP(hipMemcpy(h.f, d.f, 4 * n * sizeof(double), hipMemcpyDeviceToHost));
         TFG_HIP(hipMemcpy(h.cid, d.cid, n * sizeof(int), hipMemcpyDeviceToHost));
         TFG_HIP(hipMemcpy(h.flags, d.flags, n * sizeof(int), hipMemcpyDeviceToHost));
-        if (d.ns > 0) {
-            TFG_HIP(hipMemcpy(h.sp, d.sp, n * d.ns * sizeof(double), hipMemcpyDeviceToHost));
-            TFG_HIP(hipMemcpy(h.q, d.q, n * d.ns * sizeof(double), hipMemcpyDeviceToHost));
+        if (S > 0) {
+            TFG_HIP(hipMemcpy(h.sp, d.sp, n * S * sizeof(double), hipMemcpyDeviceToHost));
+            TFG_HIP(hipMemcpy(h.q, d.q, n * S * sizeof(double), hipMemcpyDeviceToHost));
         }
+        for (size_t p = 0, ns = h.ns; ns < S && p < n; p++)   // the ensemble's species per row: the member's
+            for (size_t k = 0; k < ns; k++) {
+                h.sp[p * ns + k] = h.sp[p * S + k];
+                h.q[p * ns + k] = h.q[p * S + k];
+            }
         record_rows(e, h, 0, static_cast<int>(n));
     }
     return TFG_OK;
